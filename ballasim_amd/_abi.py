@@ -129,6 +129,7 @@ SIGNATURES = {
     "bsx_last_error": (C.c_int, [C.c_char_p, C.c_size_t]),
     "bsx_device_count": (C.c_int, [C.POINTER(C.c_int32)]),
     "bsx_math_selfcheck": (C.c_int, [C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]),
+    "bsx_math_hash": (C.c_int, [C.c_int32, C.c_uint32, C.c_uint32, C.c_uint32, C.POINTER(C.c_uint64)]),
     "bsx_params_preset": (C.c_int, [C.c_char_p, C.POINTER(Params)]),
     "bsx_preset_names": (C.c_int, [C.c_char_p, C.c_size_t]),
     "bsx_params_validate": (C.c_int, [C.POINTER(Params)]),

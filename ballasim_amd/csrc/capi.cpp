@@ -127,6 +127,20 @@ int bsx_math_selfcheck(uint64_t* log_violations, uint64_t* log_hash) {
   });
 }
 
+int bsx_math_hash(int32_t fn, uint32_t first, uint32_t last, uint32_t stride, uint64_t* hash) {
+  return guarded([&] {
+    need_ptr(hash, "hash");
+    int n = 0;
+    if (hipGetDeviceCount(&n) != hipSuccess || n < 1) throw std::runtime_error("bsx_math_hash: no HIP device");
+    bsx::DeviceBuffer d;
+    unsigned long long h = 0;
+    bsx::hip_check(bsx::launch_math_hash(fn, first, last, stride, static_cast<unsigned long long*>(d.ensure(8)), nullptr),
+                   "bsx_math_hash");
+    bsx::hip_check(hipMemcpy(&h, d.get(), 8, hipMemcpyDeviceToHost), "bsx_math_hash");
+    *hash = h;
+  });
+}
+
 int bsx_params_preset(const char* name, bsx_params* out) {
   return guarded([&] {
     need_ptr(name, "name");

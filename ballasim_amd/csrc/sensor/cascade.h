@@ -20,26 +20,40 @@
 namespace bsx {
 namespace cascade {
 
-// g(u) = c0 + c1 u + c2 u^2 + c3 u^3 + C0 R_j(a0 u) + C1 R_j(a1 u), u in seconds (j = order).
-struct ExpCubic {
+// g(u) = c0 + c1 u + c2 u^2 + c3 u^3 + C0 E(a0 u) + C1 E(a1 u), u in seconds: E the residual exponential
+// R_kJ when resid is set, else e^-y (the order a compile-time constant, so that the residual's series
+// divides by constants).
+template <int kJ>
+struct ExpCubicT {
   float c[4];
   float C[2];
   float a[2];
-  int order;
+  bool resid;
 
   BSX_HD BSX_INLINE float poly(float u) const { return c[0] + u * (c[1] + u * (c[2] + u * c[3])); }
   BSX_HD BSX_INLINE float term(int i, float u) const {
-    return C[i] == 0.0f ? 0.0f : C[i] * pm::resid_exp(order, a[i] * u);
+    if (C[i] == 0.0f) return 0.0f;
+    const float y = a[i] * u;
+    return C[i] * (resid ? pm::resid_exp<kJ>(y) : pm::exp(-y));
   }
   BSX_HD BSX_INLINE float operator()(float u) const { return poly(u) + term(0, u) + term(1, u); }
   BSX_HD BSX_INLINE float operator()(float u, float r0, float r1) const {
     return poly(u) + (C[0] == 0.0f ? 0.0f : C[0] * r0) + (C[1] == 0.0f ? 0.0f : C[1] * r1);
   }
 };
+using ExpCubic = ExpCubicT<4>;
 
-BSX_HD BSX_INLINE ExpCubic derivative(const ExpCubic& g, int n) {
-  ExpCubic d = g;
-  for (int k = 0; k < n; ++k) {
+// The kN-th derivative: a residual R_4 becomes R_(4 - kN), an exponential stays one.
+template <int kN>
+BSX_HD BSX_INLINE ExpCubicT<4 - kN> derivative(const ExpCubic& g) {
+  ExpCubicT<4 - kN> d;
+  for (int m = 0; m < 4; ++m) d.c[m] = g.c[m];
+  for (int i = 0; i < 2; ++i) {
+    d.C[i] = g.C[i];
+    d.a[i] = g.a[i];
+  }
+  d.resid = g.resid;
+  for (int k = 0; k < kN; ++k) {
     d.c[0] = d.c[1];
     d.c[1] = 2.0f * d.c[2];
     d.c[2] = 3.0f * d.c[3];
@@ -47,7 +61,6 @@ BSX_HD BSX_INLINE ExpCubic derivative(const ExpCubic& g, int n) {
     d.C[0] = -d.a[0] * d.C[0];
     d.C[1] = -d.a[1] * d.C[1];
   }
-  d.order = g.order > n ? g.order - n : 0;
   return d;
 }
 
@@ -62,11 +75,15 @@ BSX_HD BSX_INLINE ExpCubic shifted(const ExpCubic& g, float d) {
     if (g.C[i] == 0.0f) continue;
     const float ad = g.a[i] * d;
     s.C[i] = g.C[i] * pm::exp(-ad);
+    if (!g.resid) continue;
     float coef = g.C[i];
-    for (int m = 0; m < g.order; ++m) {
-      s.c[m] = s.c[m] + coef * pm::resid_exp(g.order - m, ad);
-      coef = coef * (-g.a[i]) / static_cast<float>(m + 1);
-    }
+    s.c[0] = s.c[0] + coef * pm::resid_exp<4>(ad);
+    coef = coef * (-g.a[i]);
+    s.c[1] = s.c[1] + coef * pm::resid_exp<3>(ad);
+    coef = coef * (-g.a[i]) / 2.0f;
+    s.c[2] = s.c[2] + coef * pm::resid_exp<2>(ad);
+    coef = pm::div_by_any<3>(coef * (-g.a[i]));
+    s.c[3] = s.c[3] + coef * pm::resid_exp<1>(ad);
   }
   return s;
 }
@@ -83,14 +100,15 @@ BSX_HD BSX_INLINE Range cubic_range(const float* c, float u0, float u1) {
   const float q2 = (c[2] + u0 * (3.0f * c[3])) * (w * w);
   const float q3 = c[3] * (w * w * w);
   const float b0 = q0;
-  const float b1 = q0 + q1 / 3.0f;
-  const float b2 = q0 + (2.0f * q1 + q2) / 3.0f;
+  const float b1 = q0 + pm::div_by_any<3>(q1);
+  const float b2 = q0 + pm::div_by_any<3>(2.0f * q1 + q2);
   const float b3 = q0 + q1 + q2 + q3;
   return {vmin(vmin(b0, b1), vmin(b2, b3)), vmax(vmax(b0, b1), vmax(b2, b3))};
 }
 
 // Conservative range of g: the cubic's hull plus each monotone exponential term's end values.
-BSX_HD BSX_INLINE Range range(const ExpCubic& g, float u0, float u1) {
+template <int kJ>
+BSX_HD BSX_INLINE Range range(const ExpCubicT<kJ>& g, float u0, float u1) {
   Range r = cubic_range(g.c, u0, u1);
   for (int i = 0; i < 2; ++i) {
     if (g.C[i] == 0.0f) continue;
@@ -110,7 +128,8 @@ BSX_HD BSX_INLINE float root_tolerance(float hi) { return vmax(1e-11f, 16.0f * 0
 
 // ITP root of f on [a, b] with f(a) f(b) < 0 (Oliveira and Takahashi 2020; kappa1 = 0.2 / (b - a),
 // kappa2 = 2, n0 = 1).
-BSX_HD BSX_INLINE float itp_root(const ExpCubic& f, float a, float b, float fa, float fb, float tol) {
+template <int kJ>
+BSX_HD BSX_INLINE float itp_root(const ExpCubicT<kJ>& f, float a, float b, float fa, float fb, float tol) {
   const float width0 = b - a;
   const float k1 = 0.2f / width0;
   int n_half = 0;
@@ -157,8 +176,8 @@ BSX_HD BSX_INLINE void level_roots(const ExpCubic& g, float lo, float hi, float 
   if constexpr (N >= 4) {
     fourth_derivative_root(g, lo, hi, out);
   } else {
-    const ExpCubic f = derivative(g, N);
-    const ExpCubic fd = derivative(g, N + 1);
+    const auto f = derivative<N>(g);
+    const auto fd = derivative<N + 1>(g);
     RootList pts;
     pts.n = 0;
     pts.v[pts.n++] = lo;
@@ -282,8 +301,8 @@ BSX_HD BSX_INLINE float gl8_pair(float kh, float I0, float dI, double xi, double
 }
 
 // z after h from z0 for I linear I0 -> I1: GL8 (P <= 1/2, with the fp32 small-slope expansion),
-// zero-order hold (slope below one ulp), Dawson (rising), erfcx (falling).
-BSX_HD BSX_INLINE float z_step(float z0, float I0, float I1, float h, float k) {
+// zero-order hold (slope below one ulp), Dawson (rising), erfcx (falling). yh: recip(h).
+BSX_HD BSX_INLINE float z_step(float z0, float I0, float I1, float h, float k, float yh) {
   const float kh = k * h;
   const float Im = 0.5f * (I0 + I1);
   const float P = kh * Im;
@@ -292,7 +311,7 @@ BSX_HD BSX_INLINE float z_step(float z0, float I0, float I1, float h, float k) {
   if (P <= 0.5f) {
     if (P > 0.0f && P * fabs_(dI) <= 2.4e-4f * Im) {
       const float x = kh * I1;
-      const float b = 0.5f * k * dI / h;
+      const float b = pm::div_with(0.5f * k * dI, h, yh);
       const float one_m_E = -pm::expm1(-x);
       const float g = 1.0f / 3.0f + x * (-0.25f + x * (0.1f + x * (-1.0f / 36.0f + x * (1.0f / 168.0f))));
       const float J = one_m_E / x * h + b * h * h * h * g;
@@ -304,10 +323,14 @@ BSX_HD BSX_INLINE float z_step(float z0, float I0, float I1, float h, float k) {
     J = J + gl8_pair(kh, I0, dI, tables::kGl8Xi[3], tables::kGl8W[3]);
     return z0 * eP + kh * J;
   }
-  if (fabs_(dI) <= 0x1p-23f * Im) return 1.0f / Im + (z0 - 1.0f / Im) * eP;
-  const float s = fabs_(dI) / h;
-  const float r = sqrt_(k / (2.0f * s));
+  if (fabs_(dI) <= 0x1p-23f * Im) {
+    const float settled = 1.0f / Im;
+    return settled + (z0 - settled) * eP;
+  }
+  const float s = pm::div_with(fabs_(dI), h, yh);
+  // r = sqrt(k / (2 s)) is half of sqrt(2 k / s): the quotients differ by a factor of 4 exactly
   const float k_over_beta = sqrt_(2.0f * k / s);
+  const float r = 0.5f * k_over_beta;
   if (dI > 0.0f) return z0 * eP + k_over_beta * (pm::dawson(r * I1) - pm::dawson(r * I0) * eP);
   constexpr double kHalfSqrtPi = 0x1.c5bf891b4ef6ap-1;  // sqrt(pi) / 2
   return z0 * eP + k_over_beta * static_cast<float>(kHalfSqrtPi) * (pm::erfcx(r * I1) - pm::erfcx(r * I0) * eP);
@@ -348,8 +371,9 @@ BSX_HD BSX_INLINE void particular(const float* c, float tau, float* b) {
 }
 
 BSX_HD BSX_INLINE float boundary_layer_factor(float P) {
-  const float p2 = P * P;
-  return vmin(p2 * p2 / 384.0f, 0.15f * P + 1.0f);
+  // (from P = 64 on the linear form is the smaller by far, and p2 p2 may overflow)
+  const float p2 = P * P, line = 0.15f * P + 1.0f;
+  return P < 64.0f ? vmin(pm::div_by<384>(p2 * p2), line) : line;
 }
 
 // Attempts the sub-step [0, h] with linear input I_a -> I_b; on success fills sub (but t_a, t_b) and
@@ -358,21 +382,23 @@ BSX_HD BSX_INLINE bool try_substep(const Consts& cc, const State& st, float i_sc
                                      bool at_floor, SubStep& sub, State& next) {
   const float k = cc.k;
   const float z_a = st.z;
-  const float z_b = z_step(z_a, I_a, I_b, h, k);
+  const float yh = pm::recip(h);
+  const float z_b = z_step(z_a, I_a, I_b, h, k, yh);
   const float I_m = 0.5f * (I_a + I_b);
-  const float z_m = z_step(z_a, I_a, I_m, 0.5f * h, k);
+  const float z_m = z_step(z_a, I_a, I_m, 0.5f * h, k, 2.0f * yh);
   const float x1a = -pm::log(z_a * i_scale), x1b = -pm::log(z_b * i_scale), x1m = -pm::log(z_m * i_scale);
-  const float da = k * (I_a - 1.0f / z_a), db = k * (I_b - 1.0f / z_b);
+  const float inv_za = pm::recip_any(z_a);
+  const float da = k * (I_a - inv_za), db = k * (I_b - pm::recip_any(z_b));
   float c[4];
-  const float delta = (x1b - x1a) / h;
+  const float delta = pm::div_with(x1b - x1a, h, yh);
   c[0] = x1a;
   c[1] = da;
-  c[2] = (3.0f * delta - 2.0f * da - db) / h;
-  c[3] = (da + db - 2.0f * delta) / (h * h);
+  c[2] = pm::div_with(3.0f * delta - 2.0f * da - db, h, yh);
+  c[3] = pm::div_with(da + db - 2.0f * delta, h * h, pm::recip(h * h));
   const float hh = 0.5f * h;
   const float mid_residual = (c[0] + hh * (c[1] + hh * (c[2] + hh * c[3]))) - x1m;
   const float P = integrated_pole(I_a, I_b, h, k);
-  const float int_ku = pm::log(z_b / z_a) + P;
+  const float int_ku = pm::log(pm::div_with(z_b, z_a, inv_za)) + P;
   const float xi0 = -pm::log(z_a * I_a) + (I_b - I_a) / (h * k * I_a * I_a);
   const float P_star = vmax(P, int_ku);
   const bool accurate = fabs_(mid_residual) <= cc.eps_accept &&
@@ -406,14 +432,14 @@ BSX_HD BSX_INLINE bool try_substep(const Consts& cc, const State& st, float i_sc
     g.c[0] = d3[0];
     g.c[1] = d3[1];
     g.c[2] = d3[2] / 2.0f;
-    g.c[3] = d3[3] / 6.0f;
-    g.order = 4;
-    r2 = pm::resid_exp(4, cc.a2 * h);
-    r3 = pm::resid_exp(4, cc.a3 * h);
-    next.s2 = d2[0] + h * (d2[1] + h * (d2[2] / 2.0f + h * (d2[3] / 6.0f))) + A2 * r2;
+    g.c[3] = pm::div_by_any<6>(d3[3]);
+    g.resid = true;
+    r2 = pm::resid_exp<4>(cc.a2 * h);
+    r3 = pm::resid_exp<4>(cc.a3 * h);
+    next.s2 = d2[0] + h * (d2[1] + h * (d2[2] / 2.0f + h * pm::div_by_any<6>(d2[3]))) + A2 * r2;
   } else {
     for (int m = 0; m < 4; ++m) g.c[m] = p3[m];
-    g.order = 0;
+    g.resid = false;
     r2 = pm::exp(-cc.a2 * h);
     if (C_s != 0.0f) r3 = pm::exp(-cc.a3 * h);
     next.s2 = p2[0] + h * (p2[1] + h * (p2[2] + h * p2[3])) + A2 * r2;
@@ -540,7 +566,7 @@ struct CascadeLane : InstantLane<kMaxG> {
         cascade::SubStep sub;
         sub.t_a = sub_ta_;
         const float h = static_cast<float>(pc_.t_b - sub_ta_) * 1e-9f;
-        sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, 0};
+        sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, false};
         sub.x1_a = sub.x1_b = x1;
         sub.int_ku = cc.k * h / z;
         sub.fallback = false;
@@ -582,7 +608,7 @@ struct CascadeLane : InstantLane<kMaxG> {
       x1 = -pm::log(z * i_scale);
       s2 = s3 = x1;
       tv = 0.0f;
-      sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, 0};
+      sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, false};
       sub.x1_a = sub.x1_b = x1;
       flags |= kFlagQuarantined;
       ++n_quarantines;
@@ -616,7 +642,7 @@ struct CascadeLane : InstantLane<kMaxG> {
         // settled under constant input: the rest of the piece in one step, no transcendental
         t_b = pc.t_b;
         const float h = static_cast<float>(pc.t_b - t_a) * 1e-9f;
-        sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, 0};
+        sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, false};
         sub.x1_a = sub.x1_b = x1;
         sub.int_ku = cc.k * h / z;
         sub.fallback = false;
@@ -644,7 +670,7 @@ struct CascadeLane : InstantLane<kMaxG> {
           x1 = -pm::log(z * i_scale);
           s2 = s3 = x1;
           tv = 0.0f;
-          sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, 0};
+          sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, false};
           sub.x1_a = sub.x1_b = x1;
           flags |= kFlagQuarantined;
           ++n_quarantines;

@@ -43,6 +43,9 @@ hipError_t launch_chain_reset(const ChainArgs& a, hipStream_t stream);
 hipError_t launch_fill_f32(float* dst, size_t n, float v, hipStream_t stream);
 // out[0] = pm::log monotonicity violations, out[1] = hash of its bits over every positive float.
 hipError_t launch_math_selfcheck(unsigned long long* out, hipStream_t stream);
+// *out = the sum of math_hash(fn, u) over u = first, first + stride, ... <= last.
+hipError_t launch_math_hash(int fn, uint32_t first, uint32_t last, uint32_t stride, unsigned long long* out,
+                            hipStream_t stream);
 // Exclusive scan of int32 counts into int64 offsets (scratch: scan_scratch_count(n) values; the
 // total lands in scratch[scan_scratch_count(n) - 1]). Defined with the scene kernels.
 size_t scan_scratch_count(size_t n);

@@ -4,6 +4,7 @@
 // sink (one atomic per wave and push site, consecutive slots for the active lanes).
 #include <hip/hip_runtime.h>
 
+#include "../core/math_check.h"
 #include "cascade.h"
 #include "kernels.h"
 #include "instant.h"
@@ -1222,6 +1223,16 @@ __global__ __launch_bounds__(256) void log_check_kernel(unsigned long long* out)
   }
 }
 
+__global__ __launch_bounds__(256) void math_hash_kernel(int fn, uint32_t first, uint32_t last, uint32_t stride,
+                                                        unsigned long long* out) {
+  uint64_t hash = 0;
+  const uint64_t step = static_cast<uint64_t>(gridDim.x) * blockDim.x * stride;
+  for (uint64_t u = first + static_cast<uint64_t>(blockIdx.x * blockDim.x + threadIdx.x) * stride; u <= last; u += step)
+    hash += math_hash(fn, static_cast<uint32_t>(u));
+  for (int off = 32; off > 0; off >>= 1) hash += __shfl_xor(hash, off);
+  if (__lane_id() == 0) atomicAdd(out, static_cast<unsigned long long>(hash));
+}
+
 inline dim3 grid_for(size_t n, int block) { return dim3(static_cast<unsigned>((n + block - 1) / block)); }
 
 }  // namespace
@@ -1341,6 +1352,14 @@ hipError_t launch_chain_reset(const ChainArgs& a, hipStream_t stream) {
 hipError_t launch_math_selfcheck(unsigned long long* out, hipStream_t stream) {
   fill_u64_kernel<<<1, 64, 0, stream>>>(out, 2, 0);
   log_check_kernel<<<2048, 256, 0, stream>>>(out);
+  return hipGetLastError();
+}
+
+hipError_t launch_math_hash(int fn, uint32_t first, uint32_t last, uint32_t stride, unsigned long long* out,
+                            hipStream_t stream) {
+  if (fn < 0 || fn >= kMathFunctions || stride == 0) return hipErrorInvalidValue;
+  fill_u64_kernel<<<1, 64, 0, stream>>>(out, 1, 0);
+  math_hash_kernel<<<2048, 256, 0, stream>>>(fn, first, last, stride, out);
   return hipGetLastError();
 }
 

@@ -56,13 +56,15 @@ BSX_HD BSX_INLINE void lower3_mul(const float* L, const float* x, float* y) {
 }
 
 // The cubic Hermite of n3 on a node of length h (s): values n3 at both ends, slopes a3 (n2 - n3).
+// (h is 1e-9 times a power of two.)
 BSX_HD BSX_INLINE void hermite(const float* xl, const float* xr, float a3, float h, float* c) {
   const float dl = a3 * (xl[1] - xl[2]), dr = a3 * (xr[1] - xr[2]);
-  const float delta = (xr[2] - xl[2]) / h;
+  const float yh = pm::recip(h);
+  const float delta = pm::div_with(xr[2] - xl[2], h, yh);
   c[0] = xl[2];
   c[1] = dl;
-  c[2] = (3.0f * delta - 2.0f * dl - dr) / h;
-  c[3] = (dl + dr - 2.0f * delta) / (h * h);
+  c[2] = pm::div_with(3.0f * delta - 2.0f * dl - dr, h, yh);
+  c[3] = pm::div_with(dl + dr - 2.0f * delta, h * h, pm::recip(h * h));
 }
 
 BSX_HD BSX_INLINE float hermite_at(const float* c, float u) { return c[0] + u * (c[1] + u * (c[2] + u * c[3])); }
@@ -239,7 +241,7 @@ struct NoiseLane : CascadeLane<kMaxG> {
       float zz = z, int_kI = 0.0f;
       while (true) {
         const float h = static_cast<float>(pc.t_b - pc.t_a) * 1e-9f;
-        if (!(pc.I_a == pc.I_b && fabs_(zz * pc.I_a - 1.0f) <= cc.eps_drop)) zz = cascade::z_step(zz, pc.I_a, pc.I_b, h, cc.k);
+        if (!(pc.I_a == pc.I_b && fabs_(zz * pc.I_a - 1.0f) <= cc.eps_drop)) zz = cascade::z_step(zz, pc.I_a, pc.I_b, h, cc.k, pm::recip(h));
         int_kI = int_kI + cascade::integrated_pole(pc.I_a, pc.I_b, h, cc.k);
         if (pc.t_b >= tc1) break;
         pc = piece(pc.t_b, tc1);
@@ -469,7 +471,7 @@ struct NoiseLane : CascadeLane<kMaxG> {
     cascade::SubStep sub;
     sub.t_a = t;
     sub.t_b = tc1;
-    sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, 0};
+    sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, false};
     sub.int_ku = cc.k * (static_cast<float>(tc1 - t) * 1e-9f) / z;
     const int64_t lo = vmax(t_search, t);
     if (lo < tc1 && may_cross(delta_fn(sub, lo, hc0, t), lo, tc1, lo, margin0)) {
