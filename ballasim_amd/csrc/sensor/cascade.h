@@ -282,8 +282,16 @@ BSX_HD BSX_INLINE Hit search(const ExpCubic& delta, int64_t e0, int64_t e1, int6
   RootList crit;
   crit.n = 0;
   if (u_hi > u_lo) crit = critical_points(delta, u_lo, u_hi);
-  const int64_t k_on = on ? first_firing(gon, crit, k_lo, k_hi) : -1;
-  const int64_t k_off = off ? first_firing(goff, crit, k_lo, k_hi) : -1;
+  int64_t k_on = -1, k_off = -1;
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma nounroll
+#endif
+  for (int side = 0; side < 2; ++side) {  // (one copy of the code for both levels)
+    if (!(side == 0 ? on : off)) continue;
+    const int64_t at = first_firing(side == 0 ? gon : goff, crit, k_lo, k_hi);
+    if (side == 0) k_on = at;
+    else k_off = at;
+  }
   if (k_on < 0 && k_off < 0) return none;
   if (k_off < 0 || (k_on >= 0 && k_on <= k_off)) return {true, true, e0 + k_on};
   return {true, false, e0 + k_off};
@@ -300,9 +308,17 @@ BSX_HD BSX_INLINE float gl8_pair(float kh, float I0, float dI, double xi, double
   return static_cast<float>(w) * (pm::exp(-g_lo) + pm::exp(-g_hi));
 }
 
-// z after h from z0 for I linear I0 -> I1: GL8 (P <= 1/2, with the fp32 small-slope expansion),
-// zero-order hold (slope below one ulp), Dawson (rising), erfcx (falling). yh: recip(h).
-BSX_HD BSX_INLINE float z_step(float z0, float I0, float I1, float h, float k, float yh) {
+// z after h from z0 for I linear I0 -> I1, as an affine function of z0 whose coefficients hold all the
+// transcendental work: z0 decay + add, or (hold) add + (z0 - add) decay.
+struct ZStep {
+  float decay, add;
+  bool hold;
+  BSX_HD BSX_INLINE float operator()(float z0) const { return hold ? add + (z0 - add) * decay : z0 * decay + add; }
+};
+
+// GL8 (P <= 1/2, with the fp32 small-slope expansion), zero-order hold (slope below one ulp), Dawson
+// (rising), erfcx (falling). yh: recip(h).
+BSX_HD BSX_INLINE ZStep z_step(float I0, float I1, float h, float k, float yh) {
   const float kh = k * h;
   const float Im = 0.5f * (I0 + I1);
   const float P = kh * Im;
@@ -315,25 +331,22 @@ BSX_HD BSX_INLINE float z_step(float z0, float I0, float I1, float h, float k, f
       const float one_m_E = -pm::expm1(-x);
       const float g = 1.0f / 3.0f + x * (-0.25f + x * (0.1f + x * (-1.0f / 36.0f + x * (1.0f / 168.0f))));
       const float J = one_m_E / x * h + b * h * h * h * g;
-      return z0 * eP + k * J;
+      return {eP, k * J, false};
     }
     float J = gl8_pair(kh, I0, dI, tables::kGl8Xi[0], tables::kGl8W[0]);
     J = J + gl8_pair(kh, I0, dI, tables::kGl8Xi[1], tables::kGl8W[1]);
     J = J + gl8_pair(kh, I0, dI, tables::kGl8Xi[2], tables::kGl8W[2]);
     J = J + gl8_pair(kh, I0, dI, tables::kGl8Xi[3], tables::kGl8W[3]);
-    return z0 * eP + kh * J;
+    return {eP, kh * J, false};
   }
-  if (fabs_(dI) <= 0x1p-23f * Im) {
-    const float settled = 1.0f / Im;
-    return settled + (z0 - settled) * eP;
-  }
+  if (fabs_(dI) <= 0x1p-23f * Im) return {eP, 1.0f / Im, true};
   const float s = pm::div_with(fabs_(dI), h, yh);
   // r = sqrt(k / (2 s)) is half of sqrt(2 k / s): the quotients differ by a factor of 4 exactly
   const float k_over_beta = sqrt_(2.0f * k / s);
   const float r = 0.5f * k_over_beta;
-  if (dI > 0.0f) return z0 * eP + k_over_beta * (pm::dawson(r * I1) - pm::dawson(r * I0) * eP);
+  if (dI > 0.0f) return {eP, k_over_beta * (pm::dawson(r * I1) - pm::dawson(r * I0) * eP), false};
   constexpr double kHalfSqrtPi = 0x1.c5bf891b4ef6ap-1;  // sqrt(pi) / 2
-  return z0 * eP + k_over_beta * static_cast<float>(kHalfSqrtPi) * (pm::erfcx(r * I1) - pm::erfcx(r * I0) * eP);
+  return {eP, k_over_beta * static_cast<float>(kHalfSqrtPi) * (pm::erfcx(r * I1) - pm::erfcx(r * I0) * eP), false};
 }
 
 // ---- Sub-steps -----------------------------------------------------------------------------------
@@ -359,6 +372,7 @@ struct Piece {
   float I_a, I_b;
   BSX_HD BSX_INLINE float at(int64_t t) const {
     if (t == t_b) return I_b;
+    if (t == t_a) return I_a;
     return I_a + (I_b - I_a) * (static_cast<float>(t - t_a) / static_cast<float>(t_b - t_a));
   }
 };
@@ -376,16 +390,42 @@ BSX_HD BSX_INLINE float boundary_layer_factor(float P) {
   return P < 64.0f ? vmin(pm::div_by<384>(p2 * p2), line) : line;
 }
 
-// Attempts the sub-step [0, h] with linear input I_a -> I_b; on success fills sub (but t_a, t_b) and
-// next. at_floor forces acceptance (1 ns).
+// What a sub-step try of [0, h] with linear input I_a -> I_b needs apart from the pixel's state: stage 1
+// over h and over h / 2, and the free modes' factors over h (R_4 of a h when the sub-step is of residual
+// form, else e^(-a h)).
+struct TryCoef {
+  ZStep full, half;
+  float r2, r3;
+};
+
+BSX_HD BSX_INLINE bool residual_form(const Consts& cc, float h) { return vmax(cc.a2, cc.a3) * h <= 1.0f; }
+
+BSX_HD BSX_INLINE TryCoef try_coef(const Consts& cc, float I_a, float I_b, float h) {
+  TryCoef q;
+  const float yh = pm::recip(h);
+  q.full = z_step(I_a, I_b, h, cc.k, yh);
+  q.half = z_step(I_a, 0.5f * (I_a + I_b), 0.5f * h, cc.k, 2.0f * yh);
+  const float y2 = cc.a2 * h, y3 = cc.a3 * h;
+  const bool resid = residual_form(cc, h);
+  q.r2 = resid ? pm::resid_exp<4>(y2) : pm::exp(-y2);
+  q.r3 = resid ? pm::resid_exp<4>(y3) : pm::exp(-y3);
+  return q;
+}
+
+// The range of the comparator input over an accepted sub-step up to roundings (the cubic's hull and the
+// free modes' end values).
+struct Hull {
+  float lo, hi;
+};
+
+// Attempts the sub-step [0, h] with linear input I_a -> I_b; on success fills sub (but t_a, t_b), next and
+// hull. at_floor forces acceptance (1 ns).
 BSX_HD BSX_INLINE bool try_substep(const Consts& cc, const State& st, float i_scale, float I_a, float I_b, float h,
-                                     bool at_floor, SubStep& sub, State& next) {
+                                     bool at_floor, const TryCoef& q, SubStep& sub, State& next, Hull& hull) {
   const float k = cc.k;
   const float z_a = st.z;
   const float yh = pm::recip(h);
-  const float z_b = z_step(z_a, I_a, I_b, h, k, yh);
-  const float I_m = 0.5f * (I_a + I_b);
-  const float z_m = z_step(z_a, I_a, I_m, 0.5f * h, k, 2.0f * yh);
+  const float z_b = q.full(z_a), z_m = q.half(z_a);
   const float x1a = -pm::log(z_a * i_scale), x1b = -pm::log(z_b * i_scale), x1m = -pm::log(z_m * i_scale);
   const float inv_za = pm::recip_any(z_a);
   const float da = k * (I_a - inv_za), db = k * (I_b - pm::recip_any(z_b));
@@ -404,8 +444,8 @@ BSX_HD BSX_INLINE bool try_substep(const Consts& cc, const State& st, float i_sc
   const bool accurate = fabs_(mid_residual) <= cc.eps_accept &&
                         fabs_(xi0) * boundary_layer_factor(P_star) <= cc.eps_accept;
   const bool linear = fabs_(c[2]) * h * h + fabs_(c[3]) * h * h * h <= cc.eps_drop;
-  const bool residual_form = vmax(cc.a2, cc.a3) * h <= 1.0f;
-  const bool conditioned = residual_form || linear || 2.0f * vmin(cc.a2, cc.a3) * h >= 1.0f;
+  const bool resid = residual_form(cc, h);
+  const bool conditioned = resid || linear || 2.0f * vmin(cc.a2, cc.a3) * h >= 1.0f;
   if (!at_floor && !(accurate && conditioned)) return false;
   float p2[4], p3[4];
   particular(c, cc.tau_o, p2);
@@ -414,13 +454,13 @@ BSX_HD BSX_INLINE bool try_substep(const Consts& cc, const State& st, float i_sc
   const float A3 = st.s3 - p3[0];
   const float C_o = A2 * cc.a3 / (cc.a3 - cc.a2);
   const float C_s = A3 - C_o;
-  float r2, r3 = 0.0f;
+  const float r2 = q.r2, r3 = resid || C_s != 0.0f ? q.r3 : 0.0f;
   ExpCubic& g = sub.s3;
   g.a[0] = cc.a2;
   g.a[1] = cc.a3;
   g.C[0] = C_o;
   g.C[1] = C_s;
-  if (residual_form) {
+  if (resid) {
     const float d1[4] = {c[0], c[1], 2.0f * c[2], 6.0f * c[3]};
     float d2[4], d3[4];
     d2[0] = st.s2;
@@ -434,22 +474,25 @@ BSX_HD BSX_INLINE bool try_substep(const Consts& cc, const State& st, float i_sc
     g.c[2] = d3[2] / 2.0f;
     g.c[3] = pm::div_by_any<6>(d3[3]);
     g.resid = true;
-    r2 = pm::resid_exp<4>(cc.a2 * h);
-    r3 = pm::resid_exp<4>(cc.a3 * h);
     next.s2 = d2[0] + h * (d2[1] + h * (d2[2] / 2.0f + h * pm::div_by_any<6>(d2[3]))) + A2 * r2;
   } else {
     for (int m = 0; m < 4; ++m) g.c[m] = p3[m];
     g.resid = false;
-    r2 = pm::exp(-cc.a2 * h);
-    if (C_s != 0.0f) r3 = pm::exp(-cc.a3 * h);
     next.s2 = p2[0] + h * (p2[1] + h * (p2[2] + h * p2[3])) + A2 * r2;
   }
   next.s3 = g(h, r2, r3);
   next.z = z_b;
-  if (fabs_(g.C[0]) * (residual_form ? r2 : 1.0f) <= cc.eps_drop &&
-      fabs_(g.C[1]) * (residual_form ? r3 : 1.0f) <= cc.eps_drop) {
+  if (fabs_(g.C[0]) * (resid ? r2 : 1.0f) <= cc.eps_drop &&
+      fabs_(g.C[1]) * (resid ? r3 : 1.0f) <= cc.eps_drop) {
     g.C[0] = 0.0f;
     g.C[1] = 0.0f;
+  }
+  {
+    const float e1 = g.c[1] * h, e2 = g.c[2] * h * h, e3 = g.c[3] * h * h * h;
+    const float b1 = e1 * (1.0f / 3.0f), b2 = (2.0f * e1 + e2) * (1.0f / 3.0f), b3 = e1 + e2 + e3;
+    const float s0 = resid ? 0.0f : g.C[0], s1 = resid ? 0.0f : g.C[1], f0 = g.C[0] * r2, f1 = g.C[1] * r3;
+    hull.lo = g.c[0] + vmin(vmin(0.0f, b1), vmin(b2, b3)) + vmin(s0, f0) + vmin(s1, f1);
+    hull.hi = g.c[0] + vmax(vmax(0.0f, b1), vmax(b2, b3)) + vmax(s0, f0) + vmax(s1, f1);
   }
   sub.x1_a = x1a;
   sub.x1_b = x1b;
@@ -466,8 +509,8 @@ BSX_HD BSX_INLINE bool settled(const Consts& cc, const State& st, float x1, floa
 
 // One pixel's cascade call: InstantLane's cursor, photocurrent and fire, plus the cascade state.
 template <int kMaxG>
-struct CascadeLane : InstantLane<kMaxG> {
-  using Base = InstantLane<kMaxG>;
+struct CascadeLane : InstantLane<kMaxG, 2> {
+  using Base = InstantLane<kMaxG, 2>;
   using Base::blind_until;
   using Base::dark;
   using Base::eps_ci;
@@ -505,111 +548,204 @@ struct CascadeLane : InstantLane<kMaxG> {
     return g;
   }
 
-  BSX_HD BSX_INLINE float s3_at(const cascade::SubStep& sub, int64_t t) const {
-    return sub.s3(static_cast<float>(t - sub.t_a) * 1e-9f);
-  }
-
-  // The plain comparator on one sub-step: releases, then first crossings until none is left.
-  template <class Sink>
-  BSX_HD BSX_INLINE void compare(const cascade::SubStep& sub, Sink& sink) {
-    while (true) {
-      if (blind_until != kNotBlind) {
-        if (blind_until >= sub.t_b) return;
-        const int64_t t = blind_until;
-        this->set_reference(t, s3_at(sub, t), 0.0f, -eps_ci);
-        blind_until = kNotBlind;
-      }
-      const int64_t lo = vmax(t_search, sub.t_a);
-      if (lo >= sub.t_b) return;
-      ++n_leaves;
-      const cascade::ExpCubic d = delta_fn(sub, lo);
-      if (!cascade::may_cross(d, lo, sub.t_b, lo, theta_on, theta_off)) {
-        t_search = vmax(t_search, sub.t_b);
-        return;
-      }
-      const cascade::Hit hit = cascade::search(d, lo, sub.t_b, lo, theta_on, theta_off);
-      if (!hit.found) {
-        t_search = vmax(t_search, sub.t_b);
-        return;
-      }
-      this->fire(hit.t, hit.on, s3_at(sub, hit.t), 0.0f, sink);
-    }
-  }
-
-  // The sub-steps of one linear piece as a resumable machine, so that a wave's lanes can share each
-  // sub-step attempt whatever piece or segment they are in: piece_begin(pc); then piece_prepare(cmp)
-  // runs the settled sub-steps (each followed by cmp) and opens the next sub-step's first try, and
-  // returns false once the piece is done; piece_attempt(cmp) makes one try_substep and, on success,
-  // commits the sub-step and runs the comparator on it (cmp(sub): the plain one, or the noise lane's
-  // tree comparator). Each lane makes the same steps in the same order as a loop over the piece.
+  // The plain comparator on one sub-step (releases, then first crossings until none is left), split for a
+  // wave's lanes: compare_quick decides the sub-steps on which nothing happens from their hull, and
+  // compare_exact makes one step of the comparator on the others (the release due, then one search and its
+  // event), after which compare_quick is asked again.
+  //
+  // Times inside a piece are kept as 32-bit offsets from its start (a piece spans at most 2^23 ns).
   cascade::Piece pc_;
-  int64_t sub_ta_, sub_tb_, h_hint_;
-  float sub_Ia_;
-  bool attempting_;
+  cascade::ExpCubic s3_fn_;  // the sub-step under comparison: s3 from cmp_a_, its end, its hull
+  int32_t cmp_a_, cmp_b_;
+  cascade::Hull hull_;
 
-  BSX_HD BSX_INLINE void piece_begin(const cascade::Piece& pc) {
-    pc_ = pc;
-    sub_ta_ = pc.t_a;
-    h_hint_ = 0;
-    attempting_ = false;
-  }
+  BSX_HD BSX_INLINE float s3_in(int64_t t) const { return s3_fn_(static_cast<float>(t - (pc_.t_a + cmp_a_)) * 1e-9f); }
 
-  template <class Cmp>
-  BSX_HD BSX_INLINE bool piece_prepare(Cmp&& cmp) {
-    while (!attempting_) {
-      if (!(sub_ta_ < pc_.t_b)) return false;
-      const cascade::State st{z, s2, s3};
-      sub_Ia_ = pc_.at(sub_ta_);
-      ++n_substeps;
-      if (pc_.I_a == pc_.I_b && cascade::settled(cc, st, x1, sub_Ia_)) {
-        // settled under constant input: the rest of the piece in one step, no transcendental
-        cascade::SubStep sub;
-        sub.t_a = sub_ta_;
-        const float h = static_cast<float>(pc_.t_b - sub_ta_) * 1e-9f;
-        sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, false};
-        sub.x1_a = sub.x1_b = x1;
-        sub.int_ku = cc.k * h / z;
-        sub.fallback = false;
-        ++n_settled;
-        if (tv != 0.0f) tv = tv * pm::exp(-sub.int_ku);
-        sub.t_b = pc_.t_b;
-        sub_ta_ = pc_.t_b;
-        cmp(sub);
-      } else {
-        sub_tb_ = h_hint_ > 0 ? vmin(pc_.t_b, sub_ta_ + 2 * h_hint_) : pc_.t_b;
-        attempting_ = true;
-      }
-    }
+  // True when the sub-step is finished. The hull, formed with a few more roundings than the exact test
+  // (each below 1e-6 of the terms, which stay below the levels plus 128), bounds the comparator input on
+  // the whole sub-step, so with a margin of 2^-10 no integer of it fires: the exact test or the search
+  // behind it says the same, and leaves the same state.
+  BSX_HD BSX_INLINE bool compare_quick() {
+    const int64_t t_a = pc_.t_a + cmp_a_, t_b = pc_.t_a + cmp_b_;
+    if (blind_until != kNotBlind) return blind_until >= t_b;
+    if (t_search >= t_b) return true;
+    const float base = leak * ns_to_s64<float>(t_a - t_ref) + dr_ref - s3_ref;
+    const float rise = fabs_(leak) * (static_cast<float>(cmp_b_ - cmp_a_) * 1e-9f) + 0x1p-10f;
+    if (!(hull_.hi + base + rise < theta_on && hull_.lo + base - rise > -theta_off)) return false;
+    ++n_leaves;
+    t_search = t_b;
     return true;
   }
 
-  template <class Cmp>
-  BSX_HD BSX_INLINE void piece_attempt(Cmp&& cmp) {
-    const int64_t t_a = sub_ta_, t_b = sub_tb_, h_ns = t_b - t_a;
+  template <class Sink>
+  BSX_HD BSX_INLINE void compare_exact(Sink& sink) {
+    const int64_t t_a = pc_.t_a + cmp_a_, t_b = pc_.t_a + cmp_b_;
+    if (blind_until != kNotBlind) {
+      if (blind_until >= t_b) return;
+      const int64_t t = blind_until;
+      this->set_reference(t, s3_in(t), 0.0f, -eps_ci);
+      blind_until = kNotBlind;
+    }
+    const int64_t lo = vmax(t_search, t_a);
+    if (lo >= t_b) return;
+    ++n_leaves;
+    cascade::SubStep sub;
+    sub.t_a = t_a;
+    sub.s3 = s3_fn_;
+    const cascade::Hit hit = cascade::search(delta_fn(sub, lo), lo, t_b, lo, theta_on, theta_off);
+    if (!hit.found) {
+      t_search = vmax(t_search, t_b);
+      return;
+    }
+    this->fire(hit.t, hit.on, s3_in(hit.t), 0.0f, sink);
+  }
+
+  // The call as a resumable machine over the segments, their pieces and the pieces' sub-steps, so that a
+  // wave's lanes share each kind of step whatever piece or segment they are in. start(t_end); then
+  // prepare() goes on to the next step that needs transcendentals: kFast, the first try of a piece that is
+  // a whole segment, whose coefficients phase A left in zc; kSlow, any other try; kExact, a comparator
+  // step; kFinished, after which end(). A lane makes the same steps in the same order as nested loops.
+  static constexpr int kFinished = 0, kFast = 1, kSlow = 2, kExact = 3, kMove = 4;
+  int32_t pc_end_, try_a_, try_b_, hint_;  // the piece's end, the due try, the sub-step length that went well
+  bool attempting_, comparing_, fast_;
+  // Phase A's coefficients of the segments, at the run's first sample (null: none), the open segment's
+  // and, loaded one segment ahead, the next one's.
+  const BSX_GLOBAL SegmentCoef* zc = nullptr;
+  SegmentCoef seg_coef_, next_coef_;
+
+  BSX_HD BSX_INLINE cascade::TryCoef fast_coef() const {
+    const auto step = [](float decay, float add) { return cascade::ZStep{fabs_(decay), add, (bits_of(decay) >> 31) != 0}; };
+    return {step(seg_coef_.decay, seg_coef_.add), step(seg_coef_.half_decay, seg_coef_.half_add), seg_coef_.r2,
+            seg_coef_.r3};
+  }
+
+  // The coefficients of the open segment (ta, tb, va, vb) as phase A stores them: the hold form is marked by
+  // the decay's sign.
+  BSX_HD BSX_INLINE SegmentCoef segment_coef() const {
+    const float h = static_cast<float>(tb - ta) * 1e-9f;
+    const cascade::TryCoef q = cascade::try_coef(cc, this->photocurrent_start(), this->photocurrent_end(), h);
+    const auto mark = [](const cascade::ZStep& s) { return s.hold ? float_of(bits_of(s.decay) | 0x80000000u) : s.decay; };
+    return {mark(q.full), q.full.add, mark(q.half), q.half.add, q.r2, q.r3};
+  }
+
+  // pc_.at at an offset of the piece.
+  BSX_HD BSX_INLINE float piece_at(int32_t off) const {
+    if (off == pc_end_) return pc_.I_b;
+    if (off == 0) return pc_.I_a;
+    return pc_.I_a + (pc_.I_b - pc_.I_a) * (static_cast<float>(off) / static_cast<float>(pc_end_));
+  }
+
+  BSX_HD BSX_INLINE void load_coef(int i) {
+    if (zc != nullptr && i < n) next_coef_ = zc[i];
+  }
+
+  // One step of the machine between its transcendental ones: the comparator on the last sub-step, then the
+  // piece's next sub-step (settled, or a try), a new piece first when the last is done. kMove: a settled
+  // sub-step was made (or the segment is empty), call it again.
+  BSX_HD BSX_INLINE int prepare() {
+    if (comparing_) {
+      if (!compare_quick()) return kExact;
+      comparing_ = false;
+    }
+    if (!attempting_) {
+      if (!(try_a_ < pc_end_)) {  // the piece is done
+        if (this->in_piece) this->t_cur = pc_.t_b;
+        this->in_piece = false;
+        if (this->seg_open && !(this->t_cur < this->stop)) {
+          // the segment is done: the next one starts at its end sample
+          if (tb == kNoBreakpoint) return kFinished;
+          this->seg_open = false;
+          ta = tb;
+          for (int g = 0; g < kMaxG; ++g)
+            if (g < G) va[g] = vb[g];
+        }
+        if (!this->seg_open) {
+          if (!(this->t_cur < this->t_end_)) return kFinished;
+          seg_coef_ = next_coef_;
+          load_coef(this->next_i + 1);
+          this->open_next();
+          this->stop = vmin(this->t_end_, tb);
+          this->seg_open = true;
+        }
+        const int64_t t = this->t_cur;
+        if (!(t < this->stop)) return kMove;
+        const int64_t e = vmin(this->stop, ((t >> kPlainSegmentLog2) + 1) * kPlainSegmentNs);
+        ++n_pieces;
+        pc_ = cascade::Piece{t, e, t == ta ? this->photocurrent_start() : this->photocurrent(t),
+                             e == tb ? this->photocurrent_end() : this->photocurrent(e)};
+        pc_end_ = static_cast<int32_t>(e - t);
+        try_a_ = 0;
+        hint_ = 0;
+        fast_ = zc != nullptr && t == ta && e == tb;
+        this->in_piece = true;
+      }
+      const cascade::State st{z, s2, s3};
+      ++n_substeps;
+      if (pc_.I_a == pc_.I_b && cascade::settled(cc, st, x1, piece_at(try_a_))) {
+        // settled under constant input: the rest of the piece in one step, no transcendental
+        cmp_a_ = try_a_;
+        cmp_b_ = pc_end_;
+        s3_fn_ = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, false};
+        hull_ = {s3, s3};
+        ++n_settled;
+        if (tv != 0.0f) tv = tv * pm::exp(-(cc.k * (static_cast<float>(pc_end_ - try_a_) * 1e-9f) / z));
+        try_a_ = pc_end_;
+        comparing_ = true;
+        return kMove;
+      }
+      try_b_ = hint_ > 0 ? vmin(pc_end_, try_a_ + 2 * hint_) : pc_end_;
+      attempting_ = true;
+    }
+    return fast_ ? kFast : kSlow;
+  }
+
+  // begin(t_end), with the machine at its start.
+  BSX_HD BSX_INLINE void start(int64_t t_end) {
+    this->begin(t_end);
+    attempting_ = comparing_ = false;
+    try_a_ = pc_end_ = 0;
+    load_coef(this->next_i);
+  }
+
+  // The due try (its coefficients: fast_coef(), or slow_coef() for a kSlow one).
+  BSX_HD BSX_INLINE void slow_input(float& I_a, float& I_b, float& h) const {
+    I_a = piece_at(try_a_);
+    I_b = piece_at(try_b_);
+    h = static_cast<float>(try_b_ - try_a_) * 1e-9f;
+  }
+  BSX_HD BSX_INLINE cascade::TryCoef slow_coef() const {
+    float I_a, I_b, h;
+    slow_input(I_a, I_b, h);
+    return cascade::try_coef(cc, I_a, I_b, h);
+  }
+
+  BSX_HD BSX_INLINE void attempt(const cascade::TryCoef& q) {
+    const int32_t a = try_a_, b = try_b_, h_ns = b - a;
     const cascade::State st{z, s2, s3};
     cascade::State next{0.0f, 0.0f, 0.0f};
     cascade::SubStep sub;
     ++n_attempts;
-    if (!cascade::try_substep(cc, st, i_scale, sub_Ia_, pc_.at(t_b), static_cast<float>(h_ns) * 1e-9f, h_ns <= 1, sub,
-                              next)) {
-      sub_tb_ = t_a + h_ns / 2;
+    fast_ = false;
+    if (!cascade::try_substep(cc, st, i_scale, piece_at(a), piece_at(b), static_cast<float>(h_ns) * 1e-9f, h_ns <= 1, q,
+                              sub, next, hull_)) {
+      try_b_ = a + h_ns / 2;
       return;
     }
     attempting_ = false;
-    if (t_b < pc_.t_b || h_hint_ > 0) h_hint_ = t_b - t_a;
+    comparing_ = true;
+    if (b < pc_end_ || hint_ > 0) hint_ = h_ns;
     if (sub.fallback) {
       flags |= kFlagSolverFallback;
       ++n_fallbacks;
     }
     if (!(next.z - next.z == 0.0f && next.z > 0.0f && next.s2 - next.s2 == 0.0f && next.s3 - next.s3 == 0.0f)) {
       // quarantine: a non-finite cascade restarts at the steady state of the current input
-      const float I = pc_.at(t_b);
-      z = 1.0f / I;
+      z = 1.0f / piece_at(b);
       x1 = -pm::log(z * i_scale);
       s2 = s3 = x1;
       tv = 0.0f;
       sub.s3 = cascade::ExpCubic{{s3, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f}, {cc.a2, cc.a3}, false};
-      sub.x1_a = sub.x1_b = x1;
+      hull_ = {s3, s3};
       flags |= kFlagQuarantined;
       ++n_quarantines;
     } else {
@@ -619,10 +755,10 @@ struct CascadeLane : InstantLane<kMaxG> {
       x1 = sub.x1_b;
       tv = tv * pm::exp(-sub.int_ku) + fabs_(sub.x1_b - sub.x1_a);
     }
-    sub.t_a = t_a;
-    sub.t_b = t_b;
-    sub_ta_ = t_b;
-    cmp(sub);
+    s3_fn_ = sub.s3;
+    cmp_a_ = a;
+    cmp_b_ = b;
+    try_a_ = b;
   }
 
   // The sub-steps of one linear piece in nested loops, each followed by the comparator (cmp(sub): the
@@ -653,8 +789,10 @@ struct CascadeLane : InstantLane<kMaxG> {
         while (true) {
           const int64_t h_ns = t_b - t_a;
           ++n_attempts;
-          if (cascade::try_substep(cc, st, i_scale, I_a, pc.at(t_b), static_cast<float>(h_ns) * 1e-9f, h_ns <= 1, sub,
-                                   next))
+          const float I_b = pc.at(t_b), h = static_cast<float>(h_ns) * 1e-9f;
+          cascade::Hull hull;
+          if (cascade::try_substep(cc, st, i_scale, I_a, I_b, h, h_ns <= 1, cascade::try_coef(cc, I_a, I_b, h), sub, next,
+                                   hull))
             break;
           t_b = t_a + h_ns / 2;
         }
@@ -689,54 +827,14 @@ struct CascadeLane : InstantLane<kMaxG> {
   }
 
 
-  // The call as a resumable machine over the segments and their pieces: begin(t_end); then
-  // prepare(sink) returns kAttempt when a sub-step try is due (attempt(sink) makes it) and kFinished
-  // once the call is done; then end().
-  static constexpr int kAttempt = 1, kFinished = 2;
-
-  template <class Sink>
-  BSX_HD BSX_INLINE int prepare(Sink& sink) {
-    const auto cmp = [&](const cascade::SubStep& sub) { compare(sub, sink); };
-    while (true) {
-      if (this->in_piece) {
-        if (piece_prepare(cmp)) return kAttempt;
-        this->in_piece = false;
-        this->t_cur = pc_.t_b;
-      }
-      if (!this->seg_open) {
-        if (!(this->t_cur < this->t_end_)) return kFinished;
-        this->open_next();
-        this->stop = vmin(this->t_end_, tb);
-        this->seg_open = true;
-      }
-      if (this->t_cur < this->stop) {
-        const int64_t t = this->t_cur;
-        const int64_t e = vmin(this->stop, ((t >> kPlainSegmentLog2) + 1) * kPlainSegmentNs);
-        ++n_pieces;
-        piece_begin(cascade::Piece{t, e, this->photocurrent(t), this->photocurrent(e)});
-        this->in_piece = true;
-        continue;
-      }
-      // the segment is done: the next one starts at its end sample
-      if (tb == kNoBreakpoint) return kFinished;
-      this->seg_open = false;
-      ta = tb;
-      for (int g = 0; g < kMaxG; ++g)
-        if (g < G) va[g] = vb[g];
-    }
-  }
-
-  template <class Sink>
-  BSX_HD BSX_INLINE void attempt(Sink& sink) {
-    piece_attempt([&](const cascade::SubStep& sub) { compare(sub, sink); });
-  }
-
-  // The call: the segments of the augmented samples in order, cut at multiples of 2^23 ns, each a
-  // linear piece of photocurrent (constant waveforms); the segment ends are fetched kAhead samples ahead.
+  // The call on one lane, in order.
   template <class Sink>
   BSX_HD BSX_INLINE void advance(int64_t t_end, Sink& sink) {
-    this->begin(t_end);
-    while (prepare(sink) == kAttempt) attempt(sink);
+    start(t_end);
+    for (int due = prepare(); due != kFinished; due = prepare()) {
+      if (due == kExact) compare_exact(sink);
+      else if (due != kMove) attempt(due == kFast ? fast_coef() : slow_coef());
+    }
     this->end();
   }
 };

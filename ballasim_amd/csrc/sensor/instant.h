@@ -26,7 +26,8 @@
 
 namespace bsx {
 
-template <int kMaxG>
+// kAhead: how many segment ends are loaded ahead of the walk.
+template <int kMaxG, int kAhead = 4>
 struct InstantLane {
   // Per-pixel constants.
   uint32_t pixel;
@@ -82,6 +83,14 @@ struct InstantLane {
     float I = dark;
     for (int g = 0; g < kMaxG; ++g)
       if (g < G) I = I + scale * va[g];
+    return I;
+  }
+
+  // photocurrent(tb) of a segment with an end sample, without its interpolation: there f = 1.
+  BSX_HD BSX_INLINE float photocurrent_end() const {
+    float I = dark;
+    for (int g = 0; g < kMaxG; ++g)
+      if (g < G) I = I + scale * (va[g] + (vb[g] - va[g]));
     return I;
   }
 
@@ -619,7 +628,6 @@ struct InstantLane {
 
   // The segment ends are loaded kAhead samples ahead of the walk (raw: clamped when a segment opens),
   // so that a lane's walk through quiet segments does not wait on one load at a time.
-  static constexpr int kAhead = 4;
   int next_i;              // the input sample that ends the next segment to open
   int64_t ft[kAhead];      // ts[next_i + k] (kNoBreakpoint past the run)
   float fv[kAhead][kMaxG];

@@ -127,6 +127,13 @@ struct ScreenBlock {
   uint32_t steady;
 };
 
+// What the cascade's first try over a whole segment needs apart from the pixel's state, written by phase A
+// per segment position: stage 1 over the segment and over its first half (z -> z decay + add; a decay with
+// its sign set: z -> add + (z - add) |decay|), and the free modes' factors over it.
+struct alignas(8) SegmentCoef {
+  float decay, add, half_decay, half_add, r2, r3;
+};
+
 struct CameraDev {
   KConst kc;
   MapsDev mp;
@@ -136,6 +143,7 @@ struct CameraDev {
   const BSX_GLOBAL int64_t* pos;          // the runs' segment positions (exclusive scan of the run lengths)
   BSX_GLOBAL int* first_loud;             // per run (null: every walk from its start)
   BSX_GLOBAL ScreenBlock* screen_blocks;  // per kScreenBlock positions (null: none)
+  BSX_GLOBAL SegmentCoef* coefs;          // per segment position (cascade; null: none)
   BSX_GLOBAL float* work;                 // per run: estimated walk cost (null: no order information)
   BSX_GLOBAL RawEventDev* ev;
   unsigned long long cap;

@@ -810,10 +810,14 @@ __global__ __launch_bounds__(kInstantBlock) __attribute__((amdgpu_waves_per_eu(3
   });
 }
 
-// Estimated cost of each run's cascade walk for the heavy-first pixel order, over every segment of
-// every camera's runs: one unit per segment plus kSearchWeight per threshold's worth of
-// log-intensity change (fast logs: a schedule only). Segment j's end sample is sample j of its run,
-// so the kernel also makes the call's input check as chain_screen_kernel does.
+// Phase A of the cascade, over every segment of every camera's runs (one thread per segment position).
+// Each run's estimated walk cost for the heavy-first pixel order: one unit per segment plus kSearchWeight
+// per threshold's worth of log-intensity change (fast logs: a schedule only). Segment j's end sample is
+// sample j of its run, so the kernel also makes the call's input check as chain_screen_kernel does. And,
+// for the noise-free cascade, the segment's coefficients (SegmentCoef): the transcendental work of a
+// sub-step try that does not depend on the pixel's state, over half of a try's instructions, done here with
+// every lane busy on segments of like kind instead of in the walk, lane by lane.
+template <int kMaxG>
 __global__ __launch_bounds__(256) void chain_cost_kernel(const CameraDev* cams, int n_cams, const CallDev* call) {
   const int64_t g0 = static_cast<int64_t>(blockIdx.x) * blockDim.x;
   if (g0 >= call->n_segments) return;
@@ -830,21 +834,53 @@ __global__ __launch_bounds__(256) void chain_cost_kernel(const CameraDev* cams, 
     run = static_cast<int>(i);
     const uint32_t p = c.pixel[i];
     const float* v = c.runs.irr + c.runs.row_start[i] * kc.groups;
-    float Ia = mp.dark[p], Ib = mp.dark[p];
-    for (int g = 0; g < kc.groups; ++g) {
+    CascadeLane<kMaxG> L;
+    L.G = kc.groups;
+    L.irr_max = kc.irr_max;
+    L.dark = mp.dark[p];
+    L.scale = mp.scale[p];
+    float Ia = L.dark, Ib = L.dark;
+    for (int g = 0; g < kMaxG; ++g) {
+      if (g >= kc.groups) continue;
       const float x = v[j * kc.groups + g];
       tally.add(x, kc.irr_max);
-      Ia += mp.scale[p] * (j == 0 ? c.in.held[static_cast<int64_t>(g) * kc.n_pixels + p] : v[(j - 1) * kc.groups + g]);
-      Ib += mp.scale[p] * x;
+      const float x0 = j == 0 ? c.in.held[static_cast<int64_t>(g) * kc.n_pixels + p] : v[(j - 1) * kc.groups + g];
+      Ia += L.scale * x0;
+      Ib += L.scale * x;
+      L.va[g] = L.clampv(x0);
+      L.vb[g] = L.clampv(x);
     }
     const float theta = vmin(mp.theta_on[p], mp.theta_off[p]);
     cost = 1.0f + kSearchWeight * fabs_(__logf(Ib) - __logf(Ia)) / theta;
+    if (c.coefs != nullptr) {
+      const BSX_GLOBAL int64_t* t = c.runs.t + c.runs.row_start[i];
+      L.ta = j == 0 ? c.t_state : t[j - 1];
+      L.tb = t[j];
+      if (L.ta < L.tb) {  // (not a first sample at the model time)
+        L.cc = cascade::Consts{kc.k, kc.a2, kc.a3, kc.tau_o, kc.tau_sf, kc.eps_accept, kc.eps_drop};
+        c.coefs[q] = L.segment_coef();
+      }
+    }
   }
   if (c.work != nullptr) wave_segmented_add(c.work, run, cost);
   tally.flush(c.counters);
 }
 
-// A cascade lane's pixel p of camera cam: its constants, its run and its state, then begin(t_end).
+// A cascade lane's constants of its camera.
+template <int kMaxG>
+__device__ __forceinline__ void cascade_constants(CascadeLane<kMaxG>& L, const CameraDev* cam) {
+  const KConst& kc = cam->kc;
+  L.irr_max = kc.irr_max;
+  L.eps_ci = kc.eps_ci;
+  L.label_cut = kc.label_cut;
+  L.refractory_ns = kc.refractory_ns;
+  L.G = kc.groups;
+  L.ideal_reset = kc.ideal_reset != 0;
+  L.cc = cascade::Consts{kc.k, kc.a2, kc.a3, kc.tau_o, kc.tau_sf, kc.eps_accept, kc.eps_drop};
+  L.t_state = cam->t_state;
+}
+
+// A cascade lane's pixel p of camera cam: its maps, its run and its state, then begin(t_end).
 template <int kMaxG>
 __device__ __forceinline__ void cascade_setup(CascadeLane<kMaxG>& L, const CameraDev* cam, int p, int64_t t_end) {
   const KConst& kc = cam->kc;
@@ -857,26 +893,20 @@ __device__ __forceinline__ void cascade_setup(CascadeLane<kMaxG>& L, const Camer
   L.leak = mp.leak[p];
   L.dark = mp.dark[p];
   L.scale = mp.scale[p];
-  L.irr_max = kc.irr_max;
-  L.eps_ci = kc.eps_ci;
-  L.label_cut = kc.label_cut;
-  L.refractory_ns = kc.refractory_ns;
-  L.G = kc.groups;
-  L.ideal_reset = kc.ideal_reset != 0;
   L.hot = mp.hot[p] != 0;
-  L.cc = cascade::Consts{kc.k, kc.a2, kc.a3, kc.tau_o, kc.tau_sf, kc.eps_accept, kc.eps_drop};
   const int32_t row = runs.row_of != nullptr ? runs.row_of[p] : -1;
   if (row >= 0) {
     const int64_t start = runs.row_start[row];
     L.ts = runs.t + start;
     L.irr = runs.irr + start * kc.groups;
     L.n = runs.row_count[row];
+    L.zc = cam->coefs != nullptr ? cam->coefs + cam->pos[row] : nullptr;
   } else {
     L.ts = nullptr;
     L.irr = nullptr;
     L.n = 0;
+    L.zc = nullptr;
   }
-  L.t_state = cam->t_state;
   L.skip = L.n > 0 && L.ts[0] == L.t_state ? 1 : 0;
   for (int g = 0; g < kMaxG; ++g)
     if (g < kc.groups) L.held[g] = in.held[static_cast<int64_t>(g) * kc.n_pixels + p];
@@ -896,7 +926,7 @@ __device__ __forceinline__ void cascade_setup(CascadeLane<kMaxG>& L, const Camer
   L.shot_rate = 0.0;
   L.shot_next = INT64_MAX;
   L.shot_index = 0;
-  L.begin(t_end);
+  L.start(t_end);
 }
 
 // A finished cascade lane's end() and its pixel's new state.
@@ -937,54 +967,228 @@ __device__ __forceinline__ void cascade_count(const CameraDev* cams, int ci, Cas
   camera_add(cams, ci, 1 + kStPieces, L.n_pieces);
 }
 
-// The cascade without noise: lane i of the launch's pixel order takes pixel order[i] of its camera
-// and advances it to t_end. Each lane runs its call as a resumable machine and the wave's lanes share
-// one loop, one sub-step try per lane per turn, so that they share each try whatever piece or segment
-// each is in (a lane's own steps are those of the loops over its segments, pieces and sub-steps, in
-// order). (Lanes that take their pixels one at a time from a queue in heavy-first order measured
-// slower: 40.7 against 36.4 ms on the first 1280x720 windows.)
-template <int kMaxG>
-__device__ __forceinline__ void cascade_lane(const CameraDev* cams, int n_cams, uint32_t n_total, const uint32_t* order,
-                                             uint32_t i, int64_t t_end) {
+// The pixels a wave's lanes take in turn: positions of the launch's heavy-first order. With a queue the grid
+// is resident and persistent: the first pixels are dealt out one per wave, wave after wave, so that the
+// heaviest lie in different waves, and later ones are taken from the queue. Without one each lane takes the
+// pixel of its place.
+struct LaneFeed {
+  uint32_t n_total, wave, n_waves, dealt;
+  unsigned int* queue;
+  bool begun = false, exhausted = false;  // (uniform over the wave)
+
+  __device__ __forceinline__ LaneFeed(uint32_t n, unsigned int* q) : n_total(n), queue(q) {
+    n_waves = gridDim.x * (blockDim.x / 64);
+    wave = (blockIdx.x * blockDim.x + threadIdx.x) / 64;
+    const uint32_t each = (n + n_waves - 1) / n_waves;
+    dealt = (each < 64 ? each : 64) * n_waves;
+  }
+
+  // Positions for the `wants` lanes (past n_total: none). Called by every lane of the wave.
+  __device__ __forceinline__ uint32_t take(bool wants) {
+    const uint32_t lane = __lane_id();
+    if (exhausted) return 0xffffffffu;
+    if (queue == nullptr) {
+      exhausted = true;
+      return wave * 64 + lane;
+    }
+    if (!begun) {
+      begun = true;
+      exhausted = dealt >= n_total;
+      return lane * n_waves < dealt ? lane * n_waves + wave : 0xffffffffu;
+    }
+    const unsigned long long waiting = __ballot(wants);
+    uint32_t first = 0;
+    if (lane == 0) first = atomicAdd(queue, static_cast<unsigned int>(__popcll(waiting)));
+    first = dealt + __shfl(first, 0);
+    exhausted = first + static_cast<uint32_t>(__popcll(waiting)) >= n_total;
+    return first + static_cast<uint32_t>(__popcll(waiting & ((1ull << lane) - 1ull)));
+  }
+};
+
+// The coefficients of the sub-step tries [0, h] with input Ia -> Ib that the lanes of `tries` are due
+// (cascade::try_coef, the same steps), worked out by the whole wave: four lanes share a try, sixteen tries at
+// a time. Lanes 0 and 1 of a quad take stage 1 over h, lanes 2 and 3 over h / 2; of the two, each evaluates one
+// of the step's two special functions (or half of its Gauss-Legendre nodes), and lanes 0 and 1 one free mode
+// each. A try alone in its wave then takes the time of one special function instead of four. (Slow tries were
+// 30 % of the 1280x720 window's walk, 8 lanes at a time at 11,700 cycles; host_ragged's, 12 lanes, 9,900.)
+// Called by every lane of the wave; returns the lane's own try's (lanes of `tries`).
+template <bool kOne>
+__device__ __forceinline__ cascade::TryCoef wave_try_coef(unsigned long long tries, float Ia, float Ib, float h,
+                                                          const cascade::Consts& cc) {
+  const int lane = __lane_id(), role = lane & 3;
+  const bool half = role >= 2, second = (role & 1) != 0;
+  cascade::TryCoef out{};
+  while (tries != 0) {
+    int src = 0, rank = -1;  // the quad's try; this lane's own rank in the round
+    for (int r = 0; r < 16 && tries != 0; ++r) {
+      const int b = __ffsll(static_cast<long long>(tries)) - 1;
+      tries &= tries - 1;
+      if ((lane >> 2) == r) src = b;
+      if (lane == b) rank = r;
+    }
+    const float I0 = __shfl(Ia, src), Ie = __shfl(Ib, src), hf = __shfl(h, src);
+    const float k = kOne ? cc.k : __shfl(cc.k, src);
+    const float a2 = kOne ? cc.a2 : __shfl(cc.a2, src), a3 = kOne ? cc.a3 : __shfl(cc.a3, src);
+    const float yf = pm::recip(hf);
+    const float I1 = half ? 0.5f * (I0 + Ie) : Ie, H = half ? 0.5f * hf : hf, yh = half ? 2.0f * yf : yf;
+    // cascade::z_step(I0, I1, H, k, yh), this lane's part of it
+    const float kh = k * H;
+    const float Im = 0.5f * (I0 + I1);
+    const float P = kh * Im;
+    const float eP = pm::exp(-P);
+    const float dI = I1 - I0;
+    float u = 0.0f, v = 0.0f, scale = 1.0f;  // what this lane has formed; the special functions' factor
+    enum { kWhole, kPairs, kHold, kDifference };
+    int form;
+    if (P <= 0.5f) {
+      if (P > 0.0f && P * fabs_(dI) <= 2.4e-4f * Im) {
+        const float x = kh * I1;
+        const float b = pm::div_with(0.5f * k * dI, H, yh);
+        const float one_m_E = -pm::expm1(-x);
+        const float g = 1.0f / 3.0f + x * (-0.25f + x * (0.1f + x * (-1.0f / 36.0f + x * (1.0f / 168.0f))));
+        const float J = one_m_E / x * H + b * H * H * H * g;
+        u = k * J;
+        form = kWhole;
+      } else {
+        u = cascade::gl8_pair(kh, I0, dI, second ? tables::kGl8Xi[2] : tables::kGl8Xi[0],
+                              second ? tables::kGl8W[2] : tables::kGl8W[0]);
+        v = cascade::gl8_pair(kh, I0, dI, second ? tables::kGl8Xi[3] : tables::kGl8Xi[1],
+                              second ? tables::kGl8W[3] : tables::kGl8W[1]);
+        form = kPairs;
+      }
+    } else if (fabs_(dI) <= 0x1p-23f * Im) {
+      u = 1.0f / Im;
+      form = kHold;
+    } else {
+      const float s = pm::div_with(fabs_(dI), H, yh);
+      const float k_over_beta = sqrt_(2.0f * k / s);
+      const float x = 0.5f * k_over_beta * (second ? I0 : I1);
+      if (dI > 0.0f) {
+        u = pm::dawson(x);
+        scale = k_over_beta;
+      } else {
+        constexpr double kHalfSqrtPi = 0x1.c5bf891b4ef6ap-1;  // sqrt(pi) / 2
+        u = pm::erfcx(x);
+        scale = k_over_beta * static_cast<float>(kHalfSqrtPi);
+      }
+      form = kDifference;
+    }
+    const float pu = __shfl_xor(u, 1), pv = __shfl_xor(v, 1);
+    float add = u;
+    if (form == kPairs) add = kh * (((u + v) + pu) + pv);
+    else if (form == kDifference) add = scale * (u - pu * eP);
+    const float y = (second ? a3 : a2) * hf;
+    const float mode = vmax(a2, a3) * hf <= 1.0f ? pm::resid_exp<4>(y) : pm::exp(-y);
+    // back to the try's own lane (rank < 0 reads lane 0, unused)
+    const int at = 4 * (rank < 0 ? 0 : rank);
+    const int hold = form == kHold;
+    cascade::TryCoef q;
+    q.full = cascade::ZStep{__shfl(eP, at), __shfl(add, at), __shfl(hold, at) != 0};
+    q.half = cascade::ZStep{__shfl(eP, at + 2), __shfl(add, at + 2), __shfl(hold, at + 2) != 0};
+    q.r2 = __shfl(mode, at);
+    q.r3 = __shfl(mode, at + 1);
+    if (rank >= 0) out = q;
+  }
+  return out;
+}
+
+// The cascade without noise. A wave's lanes run their pixels' calls as resumable machines
+// (CascadeLane::prepare) and share one loop: each turn takes one kind of step (a fast try, a slow one, a
+// comparator step) and makes it for every lane that is due it, so that the kinds' costs do not add up in
+// every turn; a kind with few lanes due waits for more. A lane whose pixel is done takes another (LaneFeed),
+// several lanes at a time, so that waiting leaves no lane idle; once there are none left, nothing waits.
+// (A lane's own steps are those of the loops over its segments, pieces and sub-steps, in order.)
+// kOne: the launch has one camera, whose constants the lanes then hold in scalar registers.
+constexpr int kRefillLanes = 8;   // idle lanes that take pixels together (4: as fast, 16: 1 % slower)
+constexpr int kTurnLanes = 16;    // lanes due a slow try, or a comparator step, that make its turn (on the 1280x720
+                                  // window 4: 25.0 ms, 8: 21.6, 16: 20.6, 20: 21.6)
+template <int kMaxG, bool kOne>
+__device__ __forceinline__ void cascade_lanes(const CameraDev* cams, int n_cams, uint32_t n_total, const uint32_t* order,
+                                              unsigned int* queue, int64_t t_end) {
   using Lane = CascadeLane<kMaxG>;
+  constexpr int kIdle = -1, kOut = -2;  // waiting for a pixel (the last one not saved yet); none left
+  LaneFeed feed(n_total, queue);
   Lane L;
   L.n_substeps = L.n_pieces = L.n_leaves = 0;
   L.n_attempts = L.n_settled = L.n_fallbacks = L.n_quarantines = 0;
-  int state = Lane::kFinished;
-  int ci = -1, p = 0;
-  const CameraDev* cam = cams;
-  if (i < n_total) {
-    const uint32_t g = order != nullptr ? order[i] : i;
-    ci = camera_of(cams, n_cams, g);
-    cam = cams + ci;
-    p = static_cast<int>(g - cam->base);
-  }
-  RigSink sink{cam, ci};
-  if (ci >= 0) {
-    cascade_setup(L, cam, p, t_end);
-    state = L.prepare(sink);
-  }
-  while (__ballot(state == Lane::kAttempt) != 0) {
-    if (state == Lane::kAttempt) {
-      L.attempt(sink);
-      state = L.prepare(sink);
+  int state = kIdle, ci = -1, p = 0;
+  if constexpr (kOne) cascade_constants(L, cams);
+  while (true) {
+    if (state == Lane::kMove) {
+      state = L.prepare();
+      if (state == Lane::kFinished) state = kIdle;
     }
+    const int idle = __popcll(__ballot(state == kIdle)), fast = __popcll(__ballot(state == Lane::kFast)),
+              slow = __popcll(__ballot(state == Lane::kSlow)), exact = __popcll(__ballot(state == Lane::kExact));
+    const int busy = __popcll(__ballot(state > Lane::kFinished));
+    if (idle + busy == 0) break;
+    if (idle > 0 && (busy == 0 || feed.exhausted || idle >= kRefillLanes)) {
+      // save the finished pixels and take new ones (a rig's counters are kept per pixel, as the next one's
+      // camera may be another)
+      const bool done = state == kIdle && ci >= 0;
+      if (done) cascade_store(L, kOne ? cams : cams + ci, p);
+      if constexpr (!kOne) {
+        cascade_count(cams, done ? ci : -1, L);
+        if (done) {
+          L.n_substeps = L.n_pieces = L.n_leaves = 0;
+          L.n_attempts = L.n_settled = L.n_fallbacks = L.n_quarantines = 0;
+        }
+      }
+      const uint32_t i = feed.take(state == kIdle);
+      if (state == kIdle) {
+        ci = -1;
+        state = kOut;
+        if (i < n_total) {
+          const uint32_t g = order != nullptr ? order[i] : i;
+          ci = kOne ? 0 : camera_of(cams, n_cams, g);
+          const CameraDev* cam = kOne ? cams : cams + ci;
+          p = static_cast<int>(g - cam->base);
+          if constexpr (!kOne) cascade_constants(L, cam);
+          cascade_setup(L, cam, p, t_end);
+          state = Lane::kMove;
+        }
+      }
+      continue;
+    }
+    const int batch = feed.exhausted ? 1 : kTurnLanes;
+    const int turn = exact >= batch ? Lane::kExact
+                     : slow >= batch ? Lane::kSlow
+                     : fast > 0      ? Lane::kFast
+                     : slow > 0      ? Lane::kSlow
+                                     : Lane::kExact;
+    const bool due = state == turn;
+    if (turn == Lane::kExact) {
+      if (due) {
+        RigSink sink{kOne ? cams : cams + ci, ci};
+        L.compare_exact(sink);
+      }
+    } else {
+      cascade::TryCoef q;
+      if (turn == Lane::kSlow) {
+        float Ia = 0.0f, Ib = 0.0f, h = 0.0f;
+        if (due) L.slow_input(Ia, Ib, h);
+        q = wave_try_coef<kOne>(__ballot(due), Ia, Ib, h, L.cc);
+      } else {
+        q = L.fast_coef();
+      }
+      if (due) L.attempt(q);
+    }
+    if (due) state = Lane::kMove;
   }
-  if (ci >= 0) cascade_store(L, cam, p);
-  cascade_count(cams, ci, L);
+  if constexpr (kOne) cascade_count(cams, 0, L);
 }
 
-// The cascade's helpers (sub-steps, the comparator's search) are inlined into the lane program: as
-// calls they saved and restored the caller's live registers through scratch on every sub-step attempt.
-// Two waves per SIMD (256 registers a lane) keep the occupancy the calls had, with a fifth of their
-// scratch.
-template <int kMaxG>
+// Bound by VALU issue and by the heaviest pixels' chains of steps. The helpers are inlined into the lane
+// program (as calls they saved and restored live registers through scratch on every try); 190 registers, two
+// waves per SIMD. On the 1280x720 window (97.6 M samples, 101.6 M tries) the walk takes 16.7 ms and phase A
+// with the coefficients 3.9, against 29.5 and 1.2 with one pixel per lane, each lane forming its own
+// coefficients and every turn taking every kind of step; a 346x260 window 0.69 ms against 1.40.
+template <int kMaxG, bool kOne>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void cascade_walk_kernel(const CameraDev* cams, int n_cams, uint32_t n_total,
                                                            const uint32_t* order, unsigned int* queue, WalkTuning tu,
                                                            const CallDev* call) {
   if (call_refused(cams, n_cams)) return;
-  const int64_t t_end = call->t_end;
-  walk_groups(n_total, queue, tu, [&](uint32_t i) { cascade_lane<kMaxG>(cams, n_cams, n_total, order, i, t_end); });
+  cascade_lanes<kMaxG, kOne>(cams, n_cams, n_total, order, queue, call->t_end);
 }
 
 // The cascade with its in-path noise: lane i of the launch's pixel order takes pixel order[i] of its
@@ -1260,8 +1464,10 @@ int resident_blocks(int kind, int tier, int block) {
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     static const void* const kernels[3][4] = {
-        {reinterpret_cast<const void*>(cascade_walk_kernel<1>), reinterpret_cast<const void*>(cascade_walk_kernel<2>),
-         reinterpret_cast<const void*>(cascade_walk_kernel<4>), reinterpret_cast<const void*>(cascade_walk_kernel<8>)},
+        {reinterpret_cast<const void*>(cascade_walk_kernel<1, true>),
+         reinterpret_cast<const void*>(cascade_walk_kernel<2, true>),
+         reinterpret_cast<const void*>(cascade_walk_kernel<4, true>),
+         reinterpret_cast<const void*>(cascade_walk_kernel<8, true>)},
         {reinterpret_cast<const void*>(instant_walk_kernel<1>), reinterpret_cast<const void*>(instant_walk_kernel<2>),
          reinterpret_cast<const void*>(instant_walk_kernel<4>), reinterpret_cast<const void*>(instant_walk_kernel<8>)},
         {reinterpret_cast<const void*>(noise_walk_kernel<1>), reinterpret_cast<const void*>(noise_walk_kernel<2>),
@@ -1292,7 +1498,12 @@ hipError_t launch_chain_prepare(const ChainArgs& a, hipStream_t stream) {
   if (a.seg_capacity > 0) {
     const dim3 grid = grid_for(static_cast<size_t>(a.seg_capacity), 256);
     const dim3 prep_grid = grid_for(static_cast<size_t>(a.seg_capacity), kSegmentAlign);
-    if (!a.instant) chain_cost_kernel<<<grid, 256, 0, stream>>>(a.cams, a.n_cams, a.call);
+    if (!a.instant) {
+      if (a.groups <= 1) chain_cost_kernel<1><<<grid, 256, 0, stream>>>(a.cams, a.n_cams, a.call);
+      else if (a.groups <= 2) chain_cost_kernel<2><<<grid, 256, 0, stream>>>(a.cams, a.n_cams, a.call);
+      else if (a.groups <= 4) chain_cost_kernel<4><<<grid, 256, 0, stream>>>(a.cams, a.n_cams, a.call);
+      else chain_cost_kernel<8><<<grid, 256, 0, stream>>>(a.cams, a.n_cams, a.call);
+    }
     else if (a.groups <= 1) chain_screen_kernel<1><<<prep_grid, 256, 0, stream>>>(a.cams, a.n_cams, a.call);
     else if (a.groups <= 2) chain_screen_kernel<2><<<prep_grid, 256, 0, stream>>>(a.cams, a.n_cams, a.call);
     else if (a.groups <= 4) chain_screen_kernel<4><<<prep_grid, 256, 0, stream>>>(a.cams, a.n_cams, a.call);
@@ -1310,9 +1521,12 @@ hipError_t launch_chain_prepare(const ChainArgs& a, hipStream_t stream) {
 int chain_walk_blocks(const ChainArgs& a) {
   const int block = a.tu.block;
   const unsigned full = static_cast<unsigned>((uint64_t{walk_group_count(a.n_total, a.tu)} * 64 + block - 1) / block);
-  if (a.tu.chunk <= 0 || a.queue == nullptr) return static_cast<int>(full);
+  const bool machines = !a.instant && !a.noise;  // the noise-free cascade's walk takes its pixels from the queue
+  if ((a.tu.chunk <= 0 && !machines) || a.queue == nullptr) return static_cast<int>(full);
   const int kind = a.instant ? 1 : a.noise ? 2 : 0;
-  return static_cast<int>(vmin(full, static_cast<unsigned>(resident_blocks(kind, group_tier(a.groups), block))));
+  const unsigned resident = static_cast<unsigned>(resident_blocks(kind, group_tier(a.groups), block));
+  // (lanes that take single pixels fill as many waves as there are pixels)
+  return static_cast<int>(vmin(machines ? (a.n_total + block / 64 - 1) / (block / 64) : full, resident));
 }
 
 hipError_t launch_chain_walk(const ChainArgs& a, hipStream_t stream) {
@@ -1333,10 +1547,22 @@ hipError_t launch_chain_walk(const ChainArgs& a, hipStream_t stream) {
     else if (tier == 2) BSX_WALK(noise_walk_kernel, 4);
     else BSX_WALK(noise_walk_kernel, 8);
   } else {
-    if (tier == 0) BSX_WALK(cascade_walk_kernel, 1);
-    else if (tier == 1) BSX_WALK(cascade_walk_kernel, 2);
-    else if (tier == 2) BSX_WALK(cascade_walk_kernel, 4);
-    else BSX_WALK(cascade_walk_kernel, 8);
+#define BSX_CASCADE(G)                                                                                           \
+  if (a.n_cams == 1)                                                                                             \
+    cascade_walk_kernel<G, true><<<grid, block, 0, stream>>>(a.cams, a.n_cams, a.n_total, a.perm, a.queue, a.tu, \
+                                                             a.call);                                            \
+  else                                                                                                           \
+    cascade_walk_kernel<G, false><<<grid, block, 0, stream>>>(a.cams, a.n_cams, a.n_total, a.perm, a.queue, a.tu, a.call)
+    if (tier == 0) {
+      BSX_CASCADE(1);
+    } else if (tier == 1) {
+      BSX_CASCADE(2);
+    } else if (tier == 2) {
+      BSX_CASCADE(4);
+    } else {
+      BSX_CASCADE(8);
+    }
+#undef BSX_CASCADE
   }
 #undef BSX_WALK
   return hipGetLastError();

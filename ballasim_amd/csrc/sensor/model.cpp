@@ -19,6 +19,7 @@ namespace {
 constexpr double kMaxSamplePhotocurrent_fA = 1e9;  // the reference's input clamp (src/sensor/pixel.h:97)
 constexpr uint32_t kStateMagic = 0x534e5342;      // "BSNS"
 constexpr uint32_t kStateVersion = 6;
+constexpr size_t kMaxCoefBytes = size_t{32} << 30;  // of segment coefficients per camera
 
 struct StateHeader {
   uint32_t magic, version;
@@ -531,6 +532,20 @@ CameraDev SensorModel::stage(const RunsDev& runs, const uint32_t* pixel, size_t 
   d_events_.ensure(cap_ * sizeof(RawEventDev));
   d_work_.ensure(std::max<size_t>(n_runs, 1) * sizeof(float));
   d_loud_.ensure(std::max<size_t>(n_runs, 1) * sizeof(int));
+  bool coefs = false;
+  if (!inst && !noise_ && total > 0) {
+    // the cascade's segment coefficients: 24 bytes per segment, left out (the walk then forms them itself)
+    // past kMaxCoefBytes or when the device has no room for them
+    const size_t bytes = static_cast<size_t>(total) * sizeof(SegmentCoef);
+    if (bytes <= kMaxCoefBytes) {
+      try {
+        d_coefs_.ensure(bytes);
+        coefs = true;
+      } catch (const std::runtime_error&) {
+        (void)hipGetLastError();
+      }
+    }
+  }
   if (inst) d_sblocks_.ensure((static_cast<size_t>(total) / kScreenBlock + 1) * sizeof(ScreenBlock));
   CameraDev cd{};
   cd.kc = kconst();
@@ -542,6 +557,7 @@ CameraDev SensorModel::stage(const RunsDev& runs, const uint32_t* pixel, size_t 
   cd.pos = d_pos_.as<const int64_t>();
   cd.first_loud = inst ? d_loud_.as<int>() : nullptr;
   cd.screen_blocks = inst ? d_sblocks_.as<ScreenBlock>() : nullptr;
+  cd.coefs = coefs ? d_coefs_.as<SegmentCoef>() : nullptr;
   cd.work = d_work_.as<float>();
   cd.ev = d_events_.as<RawEventDev>();
   cd.cap = cap_;

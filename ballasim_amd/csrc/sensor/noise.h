@@ -241,7 +241,7 @@ struct NoiseLane : CascadeLane<kMaxG> {
       float zz = z, int_kI = 0.0f;
       while (true) {
         const float h = static_cast<float>(pc.t_b - pc.t_a) * 1e-9f;
-        if (!(pc.I_a == pc.I_b && fabs_(zz * pc.I_a - 1.0f) <= cc.eps_drop)) zz = cascade::z_step(zz, pc.I_a, pc.I_b, h, cc.k, pm::recip(h));
+        if (!(pc.I_a == pc.I_b && fabs_(zz * pc.I_a - 1.0f) <= cc.eps_drop)) zz = cascade::z_step(pc.I_a, pc.I_b, h, cc.k, pm::recip(h))(zz);
         int_kI = int_kI + cascade::integrated_pole(pc.I_a, pc.I_b, h, cc.k);
         if (pc.t_b >= tc1) break;
         pc = piece(pc.t_b, tc1);

@@ -81,6 +81,35 @@ def test_cascade_matches_oracle(case):
         assert ks[f] == ko[f], (f, ks[f], ko[f])
 
 
+# Fewer pixels than a wave, one more than a wave, fewer lanes than pixels per wave, and more pixels than the
+# walk's resident lanes (256 CUs x 8 waves x 64), so that lanes take theirs from the queue.
+@pytest.mark.parametrize("W,H,frac", [(1, 1, 1.0), (63, 1, 1.0), (65, 1, 0.9), (131, 67, 0.5), (571, 293, 0.05)])
+def test_cascade_lanes_take_pixels(W, H, frac):
+    import ballasim_amd as bsx
+    rng = np.random.default_rng(W)
+    p = _params("prophesee_physical")
+    gpu = bsx.SensorModel(p, W, H, 5, ["constant"], 0, device="cuda")
+    ref = O.OracleModel(p.c, W, H, 5, 1, 0)
+    irr0 = np.exp(rng.normal(2.5, 1.2, size=(W * H, 1))).astype(np.float32)
+    gpu.init(0, irr0)
+    ref.init(0, irr0)
+    t = 0
+    for t1 in (2 ** 23, 2 ** 23 + 5 * 2 ** 20):
+        ids, ts, ir, offs = random_runs(rng, W * H, t, t1, frac=frac, max_n=40 if W * H < 100 else 8)
+        ev = gpu.advance(ids, ts, ir, t1, offsets=offs)
+        want, _ = ref.advance_runs(ids, ts, ir, offs, t1)
+        got = events_from_dict(ev, W)
+        i, a, b = first_difference(got, want)
+        assert len(got) == len(want) and i == len(got), f"first difference at {i}: gpu {a} oracle {b}"
+        t = t1
+    st = np.frombuffer(gpu.save_state()[56:], O.REF_STATE_DTYPE)
+    os_ = ref.states()
+    for f in ("z", "x1", "s2", "s3", "tv", "t_search", "blind_until", "flags"):
+        assert np.array_equal(st[f], os_[f]), f
+    for f in ("substeps", "substep_attempts", "settled_substeps", "leaf_intervals", "pieces"):
+        assert gpu.stats()[f] == ref.stats()[f], f
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_golden_fixture_replayed_on_gpu(name):
     import ballasim_amd as bsx
