@@ -181,6 +181,9 @@ SIGNATURES = {
     "bsx_output_destroy": (C.c_int, [P]),
     "bsx_output_window": (C.c_int, [P, C.POINTER(DeviceEvents), C.c_int64, P, P]),
     "bsx_output_flush": (C.c_int, [P, P, P]),
+    "bsx_output_window_count": (C.c_int, [P, C.POINTER(DeviceEvents), C.c_int64, P, P, P]),
+    "bsx_output_flush_count": (C.c_int, [P, P, P]),
+    "bsx_output_fetch": (C.c_int, [P, P, P]),
     "bsx_event_stream_create": (C.c_int, [C.c_size_t, P, P, C.POINTER(P)]),
     "bsx_event_stream_destroy": (C.c_int, [P]),
     "bsx_output_window_to_stream": (C.c_int, [P, C.POINTER(DeviceEvents), C.c_int64, P, P, P, P]),

@@ -655,6 +655,36 @@ int bsx_output_flush(bsx_output* o, void* stream, bsx_output_events* out) {
   });
 }
 
+int bsx_output_window_count(bsx_output* o, const bsx_device_events* events, int64_t t_w, void* stream, size_t* released,
+                            size_t* held) {
+  return guarded([&] {
+    need_ptr(events, "events");
+    need_ptr(released, "released");
+    bsx::OutputStage& s = output_of(o);
+    const bsx::OutEventDev* ev = nullptr;
+    *released = s.window_device(reinterpret_cast<const bsx::RawEventDev*>(events->data), events->count, t_w,
+                                static_cast<hipStream_t>(stream), &ev);
+    if (held != nullptr) *held = s.held();
+  });
+}
+
+int bsx_output_flush_count(bsx_output* o, void* stream, size_t* released) {
+  return guarded([&] {
+    need_ptr(released, "released");
+    const bsx::OutEventDev* ev = nullptr;
+    *released = output_of(o).flush_device(static_cast<hipStream_t>(stream), &ev);
+  });
+}
+
+int bsx_output_fetch(bsx_output* o, void* stream, const bsx_output_columns* dst) {
+  return guarded([&] {
+    need_ptr(dst, "dst");
+    output_of(o).fetch(bsx::OutputColumnsDst{dst->x, dst->y, dst->p, dst->t, dst->t_ns_rem, dst->t_reported_ns,
+                                             dst->t_cross_ns, dst->label, dst->flags},
+                       static_cast<hipStream_t>(stream));
+  });
+}
+
 int bsx_event_stream_create(size_t chunk_bytes, bsx_chunk_sink sink, void* user, bsx_event_stream** out) {
   return guarded([&] {
     need_ptr(out, "out");

@@ -43,6 +43,17 @@ struct CropBox {
   int32_t x0, y0, x1, y1;  // kept: x0 <= x < x1, y0 <= y < y1
 };
 
+// Where a fetch puts the columns of the released events (each with room for all of them).
+struct OutputColumnsDst {
+  uint16_t *x, *y;
+  uint8_t* p;
+  int64_t* t_us;
+  uint16_t* t_ns_rem;
+  int64_t *t_reported, *t_cross;
+  uint8_t* label;
+  uint16_t* flags;
+};
+
 // Output columns of released events (host copies, valid until the next call).
 struct OutputColumns {
   std::vector<uint16_t> x, y;
@@ -69,26 +80,44 @@ class OutputStage {
   size_t window_device(const RawEventDev* raw, size_t n, int64_t t_w, hipStream_t stream,
                        const OutEventDev** released);
   size_t flush_device(hipStream_t stream, const OutEventDev** released);
+  // The columns of the events the last window_device or flush_device released, into host arrays.
+  void fetch(const OutputColumnsDst& dst, hipStream_t stream);
   size_t held() const { return n_held_; }
+  ~OutputStage();
+  OutputStage(const OutputStage&) = delete;
+  OutputStage& operator=(const OutputStage&) = delete;
 
  private:
   // Sorts the total events of held_, moves those reported before cut to the front of sorted_ (their
   // count returned) and the rest back to held_.
   size_t release_sorted(size_t total, int64_t cut, hipStream_t stream);
+  // The same order by three stable digit sorts.
+  void sort_digits(size_t total, int64_t cut, int64_t tr_min, int64_t tr_max, int64_t tc_min, int64_t tc_max,
+                   hipStream_t stream);
   const OutputColumns& download(size_t m, hipStream_t stream);
-  // The window's raw events joined to the held ones; returns the total and sets *cut.
-  size_t take_window(const RawEventDev* raw, size_t n, int64_t t_w, hipStream_t stream, int64_t* cut);
-  size_t take_flush(hipStream_t stream);
+  // The n raw events joined to the held ones and scratch read back; returns the total.
+  size_t take(const RawEventDev* raw, size_t n, hipStream_t stream);
+  void read_scratch(hipStream_t stream);
+  // bytes of device memory to the pieces of host memory that dst names (in order), by way of pinned staging.
+  struct Piece {
+    char* to;
+    size_t bytes;
+  };
+  void copy_out(const char* from, const std::vector<Piece>& dst, size_t bytes, hipStream_t stream);
 
   uint32_t width_, height_;
-  int y_bits_;
+  int x_bits_, y_bits_;
   Readout readout_;
   bool crop_on_;
   CropBox crop_{};
   int64_t t_offset_us_;
   size_t n_held_ = 0;
   DeviceBuffer held_, sorted_, keys_, keys_alt_, perm_, perm_alt_, temp_, scratch_;
-  DeviceBuffer cx_, cy_, cp_, ct_, crem_, ctr_, ctc_, clab_, cfl_;
+  DeviceBuffer buckets_, columns_;
+  size_t released_ = 0;                 // at the front of sorted_, from the last call
+  unsigned long long* h_scratch_ = nullptr;  // pinned
+  char* staging_ = nullptr;             // pinned: staging_slots_ slots of kCopyBytes
+  int staging_slots_ = 0;
   OutputColumns out_;
 };
 

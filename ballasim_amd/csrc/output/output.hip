@@ -22,58 +22,20 @@ __device__ __forceinline__ uint8_t label_s1(uint8_t c) {
 constexpr uint64_t kBias = uint64_t{1} << 63;
 constexpr int kOutBlock = 256;  // threads per block of the per-event kernels
 
-__global__ void build_kernel(const RawEventDev* raw, size_t n, uint32_t width, Readout r, int crop, CropBox box,
-                             OutEventDev* out, unsigned long long* scratch) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  bool keep = false;
-  OutEventDev o{};
-  if (i < n) {
-    const RawEventDev e = raw[i];
-    const int32_t x = static_cast<int32_t>(e.pixel % width), y = static_cast<int32_t>(e.pixel / width);
-    keep = !crop || (x >= box.x0 && x < box.x1 && y >= box.y0 && y < box.y1);
-    o.t_cross = e.t_cross;
-    o.t_reported = reported_time(r, e.t_cross);
-    o.x = static_cast<uint16_t>(x);
-    o.y = static_cast<uint16_t>(y);
-    o.flags = e.flags;
-    o.p = e.polarity;
-    o.label = label_s1(e.label);
-  }
-  // block-aggregated slots, one atomic per block (the order of the kept events does not matter: the
-  // output key is unique)
-  __shared__ unsigned int wave_kept[kOutBlock / 64];
-  __shared__ unsigned long long block_base;
-  const unsigned long long mask = __ballot(keep);
-  const int lane = __lane_id(), wave = threadIdx.x >> 6;
-  if (lane == 0) wave_kept[wave] = static_cast<unsigned int>(__popcll(mask));
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long total = 0;
-    for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) total += wave_kept[w];
-    block_base = total != 0 ? atomicAdd(scratch, total) : 0;
-  }
-  __syncthreads();
-  unsigned long long base = block_base;
-  for (int w = 0; w < wave; ++w) base += wave_kept[w];
-  if (keep) out[base + __popcll(mask & ((1ull << lane) - 1ull))] = o;
+// Raw events a block takes at once: one atomic on the kept count and one set on the extremes per 2,048 events
+// (per 256 the atomics on one address set the time: 143 us and a separate 40-us pass over 2.9 M events).
+constexpr int kBuildItems = 8;
+
+__global__ void reset_kernel(unsigned long long* scratch) {
+  if (threadIdx.x < kOutScratch)
+    scratch[threadIdx.x] = threadIdx.x == kOutRepMin || threadIdx.x == kOutLagMin ? ~0ull : 0ull;
 }
 
-// The extremes of t_cross and t_reported (biased to unsigned order) over ev[0 .. n_held + scratch[0]):
-// a grid-stride loop over a bounded grid, reduced in the wave and then in the block, so that each block
-// makes one set of four atomics.
-__global__ void minmax_kernel(const OutEventDev* ev, size_t n_held, size_t n_max, unsigned long long* scratch) {
+// The extremes of the reported times and of the lags t_cross - t_reported (biased to unsigned order) of a
+// block's threads into scratch. Called by every thread of the block.
+__device__ __forceinline__ void fold_extremes(unsigned long long a, unsigned long long b, unsigned long long c,
+                                              unsigned long long d, unsigned long long* scratch) {
   __shared__ unsigned long long part[4][kOutBlock / 64];
-  const size_t n = vmin(n_held + static_cast<size_t>(scratch[0]), n_max);
-  unsigned long long a = ~0ull, b = 0ull, c = ~0ull, d = 0ull;
-  for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const unsigned long long tc = static_cast<uint64_t>(ev[i].t_cross) ^ kBias;
-    const unsigned long long tr = static_cast<uint64_t>(ev[i].t_reported) ^ kBias;
-    a = min(a, tc);
-    b = max(b, tc);
-    c = min(c, tr);
-    d = max(d, tr);
-  }
   for (int off = 32; off > 0; off >>= 1) {
     a = min(a, static_cast<unsigned long long>(__shfl_xor(a, off)));
     b = max(b, static_cast<unsigned long long>(__shfl_xor(b, off)));
@@ -96,12 +58,200 @@ __global__ void minmax_kernel(const OutEventDev* ev, size_t n_held, size_t n_max
       d = max(d, part[3][w]);
     }
     if (a != ~0ull) {
-      atomicMin(scratch + 1, a);
-      atomicMax(scratch + 2, b);
-      atomicMin(scratch + 3, c);
-      atomicMax(scratch + 4, d);
+      atomicMin(scratch + kOutRepMin, a);
+      atomicMax(scratch + kOutRepMax, b);
+      atomicMin(scratch + kOutLagMin, c);
+      atomicMax(scratch + kOutLagMax, d);
     }
   }
+}
+
+// Appends the kept raw events at held[n_held ..] and folds the extremes of the new and the held events.
+__global__ __launch_bounds__(kOutBlock) void build_kernel(const RawEventDev* raw, size_t n, uint32_t width, Readout r,
+                                                          int crop, CropBox box, OutEventDev* held, size_t n_held,
+                                                          unsigned long long* scratch) {
+  unsigned long long a = ~0ull, b = 0ull, c = ~0ull, d = 0ull;
+  const auto fold = [&](const OutEventDev& o) {
+    const unsigned long long tr = static_cast<uint64_t>(o.t_reported) ^ kBias;
+    const unsigned long long lag = static_cast<uint64_t>(o.t_cross - o.t_reported) ^ kBias;
+    a = min(a, tr);
+    b = max(b, tr);
+    c = min(c, lag);
+    d = max(d, lag);
+  };
+  for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n_held;
+       i += static_cast<size_t>(gridDim.x) * blockDim.x)
+    fold(held[i]);
+  __shared__ unsigned int kept[kBuildItems * (kOutBlock / 64)];
+  __shared__ unsigned long long block_base;
+  const int lane = __lane_id(), wave = threadIdx.x >> 6;
+  OutEventDev ev[kBuildItems];
+  unsigned long long mask[kBuildItems];
+  for (int k = 0; k < kBuildItems; ++k) {
+    const size_t i = (static_cast<size_t>(blockIdx.x) * kBuildItems + k) * kOutBlock + threadIdx.x;
+    bool keep = false;
+    OutEventDev o{};
+    if (i < n) {
+      const RawEventDev e = raw[i];
+      const int32_t x = static_cast<int32_t>(e.pixel % width), y = static_cast<int32_t>(e.pixel / width);
+      keep = !crop || (x >= box.x0 && x < box.x1 && y >= box.y0 && y < box.y1);
+      o.t_cross = e.t_cross;
+      o.t_reported = reported_time(r, e.t_cross);
+      o.x = static_cast<uint16_t>(x);
+      o.y = static_cast<uint16_t>(y);
+      o.flags = e.flags;
+      o.p = e.polarity;
+      o.label = label_s1(e.label);
+      if (keep) fold(o);
+    }
+    ev[k] = o;
+    mask[k] = __ballot(keep);
+    if (lane == 0) kept[k * (kOutBlock / 64) + wave] = static_cast<unsigned int>(__popcll(mask[k]));
+  }
+  __syncthreads();
+  // (the order of the kept events does not matter: the output key is unique)
+  if (threadIdx.x == 0) {
+    unsigned int total = 0;
+    for (int q = 0; q < kBuildItems * (kOutBlock / 64); ++q) {
+      const unsigned int w = kept[q];
+      kept[q] = total;
+      total += w;
+    }
+    block_base = total != 0 ? atomicAdd(scratch + kOutKept, static_cast<unsigned long long>(total)) : 0;
+  }
+  __syncthreads();
+  for (int k = 0; k < kBuildItems; ++k) {
+    if ((mask[k] >> lane) & 1ull)
+      held[n_held + block_base + kept[k * (kOutBlock / 64) + wave] + __popcll(mask[k] & ((1ull << lane) - 1ull))] = ev[k];
+  }
+  fold_extremes(a, b, c, d, scratch);
+}
+
+// ---- The bucket sort -----------------------------------------------------------------------------
+// The output order is the order of one integer key (OrderKey: t_reported, x, y and the lag t_cross -
+// t_reported, each less its minimum), unique per event. Its leading bits part the events into buckets of a few
+// hundred (reported times spread over the window), counted and filled with one atomic per event, and one block
+// per bucket sorts its keys in LDS and writes the events in order: four short passes whatever the key's
+// length, where the digit sort below makes ten of five kernels each (2.9 M events: 0.58 ms of kernels, and
+// 50 launches in a window of any size). Keys of more than 64 bits, and a bucket of more than kBucketCap events
+// (coarse readouts), are left to the digit sort.
+constexpr int kBucketCap = 2048;
+
+__device__ __forceinline__ uint64_t order_key(const OrderKey& k, const OutEventDev& o) {
+  return (((((static_cast<uint64_t>(o.t_reported - k.rep_min) << k.x_bits) | o.x) << k.y_bits) | o.y) << k.lag_bits) |
+         static_cast<uint64_t>((o.t_cross - o.t_reported) - k.lag_min);
+}
+
+// (clamped: an event outside the frame has a key past the others')
+__device__ __forceinline__ uint32_t bucket_of(uint64_t key, int shift, uint32_t buckets) {
+  const uint64_t b = key >> shift;
+  return b < buckets ? static_cast<uint32_t>(b) : buckets - 1;
+}
+
+__global__ __launch_bounds__(256) void bucket_count_kernel(const OutEventDev* ev, size_t n, OrderKey k, int shift,
+                                                           uint32_t buckets, uint32_t* counts) {
+  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) atomicAdd(counts + bucket_of(order_key(k, ev[i]), shift, buckets), 1u);
+}
+
+// base[b] = cursor[b] = the events of the buckets before b; the largest bucket in scratch (one block).
+__global__ __launch_bounds__(1024) void bucket_scan_kernel(const uint32_t* counts, int buckets, uint32_t* base,
+                                                           uint32_t* cursor, unsigned long long* scratch) {
+  __shared__ uint32_t wave_sum[16];
+  __shared__ uint32_t carry;
+  if (threadIdx.x == 0) carry = 0;
+  uint32_t most = 0;
+  for (int b0 = 0; b0 < buckets; b0 += 1024) {
+    __syncthreads();
+    const int b = b0 + threadIdx.x, lane = __lane_id(), wave = threadIdx.x >> 6;
+    const uint32_t v = b < buckets ? counts[b] : 0;
+    most = max(most, v);
+    uint32_t inc = v;
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t o = __shfl_up(inc, off);
+      if (lane >= off) inc += o;
+    }
+    if (lane == 63) wave_sum[wave] = inc;
+    __syncthreads();
+    uint32_t before = carry;
+    for (int w = 0; w < wave; ++w) before += wave_sum[w];
+    if (b < buckets) {
+      base[b] = before + inc - v;
+      cursor[b] = before + inc - v;
+    }
+    __syncthreads();
+    if (threadIdx.x == 1023) carry = before + inc;
+  }
+  for (int off = 32; off > 0; off >>= 1) most = max(most, static_cast<uint32_t>(__shfl_xor(most, off)));
+  if (__lane_id() == 0) atomicMax(scratch + kOutMostBucket, static_cast<unsigned long long>(most));
+}
+
+__global__ __launch_bounds__(256) void bucket_fill_kernel(const OutEventDev* ev, size_t n, OrderKey k, int shift,
+                                                          uint32_t buckets, uint32_t* cursor, uint64_t* keys, uint32_t* perm) {
+  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint64_t key = order_key(k, ev[i]);
+  const uint32_t slot = atomicAdd(cursor + bucket_of(key, shift, buckets), 1u);
+  keys[slot] = key;
+  perm[slot] = static_cast<uint32_t>(i);
+}
+
+// One block per bucket: its keys sorted in LDS (bitonic, padded to a power of two with the largest key), its
+// events written in order and those reported before cut counted. With base null the events are one bucket,
+// whose keys the block forms itself. A bucket past kBucketCap is left alone (the host sees the largest).
+__global__ __launch_bounds__(256) void bucket_sort_kernel(const OutEventDev* ev, size_t n, OrderKey k,
+                                                          const uint32_t* counts, const uint32_t* base,
+                                                          const uint64_t* keys, const uint32_t* perm, int64_t cut,
+                                                          OutEventDev* sorted, unsigned long long* scratch) {
+  __shared__ uint64_t key[kBucketCap];
+  __shared__ uint32_t idx[kBucketCap];
+  __shared__ uint32_t ready;
+  const uint32_t c = base != nullptr ? counts[blockIdx.x] : static_cast<uint32_t>(n);
+  const uint32_t first = base != nullptr ? base[blockIdx.x] : 0;
+  if (c == 0 || c > kBucketCap) return;
+  uint32_t size = 64;
+  while (size < c) size <<= 1;
+  if (threadIdx.x == 0) ready = 0;
+  for (uint32_t i = threadIdx.x; i < size; i += 256) {
+    const bool real = i < c;
+    const uint32_t e = !real ? 0u : base != nullptr ? perm[first + i] : i;
+    key[i] = !real ? ~0ull : base != nullptr ? keys[first + i] : order_key(k, ev[e]);
+    idx[i] = real ? e : 0xffffffffu;  // (a real key of all ones sorts before the padding)
+  }
+  __syncthreads();
+  for (uint32_t span = 2; span <= size; span <<= 1) {
+    for (uint32_t step = span >> 1; step > 0; step >>= 1) {
+      for (uint32_t q = threadIdx.x; q < size / 2; q += 256) {
+        const uint32_t lo = 2 * q - (q & (step - 1)), hi = lo + step;
+        const bool up = (lo & span) == 0;
+        const uint64_t ka = key[lo], kb = key[hi];
+        const uint32_t ia = idx[lo], ib = idx[hi];
+        const bool above = ka > kb || (ka == kb && ia > ib);
+        if (above == up) {
+          key[lo] = kb;
+          key[hi] = ka;
+          idx[lo] = ib;
+          idx[hi] = ia;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  uint32_t mine = 0;
+  for (uint32_t i = threadIdx.x; i < c; i += 256) {
+    const OutEventDev o = ev[idx[i]];
+    sorted[first + i] = o;
+    mine += o.t_reported < cut ? 1u : 0u;
+  }
+  for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off);
+  if (__lane_id() == 0 && mine != 0) atomicAdd(&ready, mine);
+  __syncthreads();
+  if (threadIdx.x == 0 && ready != 0) atomicAdd(scratch + kOutReady, static_cast<unsigned long long>(ready));
+}
+
+__global__ void fill_counts_kernel(uint32_t* counts, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) counts[i] = 0;
 }
 
 __global__ void keys_kernel(const OutEventDev* ev, const uint32_t* perm, uint32_t* perm_init, size_t n, int pass,
@@ -133,7 +283,7 @@ __global__ void gather_kernel(const OutEventDev* ev, const uint32_t* perm, size_
   if (threadIdx.x == 0) {
     unsigned long long total = 0;
     for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) total += wave_ready[w];
-    if (total != 0) atomicAdd(scratch + 5, total);
+    if (total != 0) atomicAdd(scratch + kOutReady, total);
   }
 }
 
@@ -239,16 +389,48 @@ inline unsigned grid(size_t n) { return static_cast<unsigned>((n + kOutBlock - 1
 }  // namespace
 
 hipError_t launch_out_build(const RawEventDev* raw, size_t n, uint32_t width, const Readout& r, bool crop,
-                            const CropBox& box, OutEventDev* out, unsigned long long* scratch, hipStream_t stream) {
-  if (n == 0) return hipSuccess;
-  build_kernel<<<grid(n), kOutBlock, 0, stream>>>(raw, n, width, r, crop ? 1 : 0, box, out, scratch);
+                            const CropBox& box, OutEventDev* held, size_t n_held, unsigned long long* scratch,
+                            hipStream_t stream) {
+  reset_kernel<<<1, 64, 0, stream>>>(scratch);
+  if (n + n_held > 0) {
+    const size_t tile = static_cast<size_t>(kOutBlock) * kBuildItems;
+    // (blocks past the new events, up to a bound, stride over the held ones)
+    const unsigned blocks = vmax(static_cast<unsigned>((n + tile - 1) / tile), vmin(grid(n_held), 512u));
+    build_kernel<<<blocks, kOutBlock, 0, stream>>>(raw, n, width, r, crop ? 1 : 0, box, held, n_held, scratch);
+  }
   return hipGetLastError();
 }
 
-hipError_t launch_out_minmax(const OutEventDev* ev, size_t n_held, size_t n_max, unsigned long long* scratch,
-                             hipStream_t stream) {
-  if (n_max == 0) return hipSuccess;
-  minmax_kernel<<<vmin(grid(n_max), 1024u), kOutBlock, 0, stream>>>(ev, n_held, n_max, scratch);
+int out_bucket_bits(size_t n) {
+  int b = 0;
+  while (n > kBucketCap && (n >> b) > 512 && b < kMaxBucketBits) ++b;
+  return b;
+}
+
+size_t out_bucket_cap() { return kBucketCap; }
+
+hipError_t launch_out_buckets(const OutEventDev* ev, size_t n, const OrderKey& k, int bucket_bits, int64_t cut,
+                              uint32_t* words, uint64_t* keys, uint32_t* perm, OutEventDev* sorted,
+                              unsigned long long* scratch, hipStream_t stream) {
+  if (n == 0) return hipSuccess;
+  if (bucket_bits == 0) {
+    if (n > kBucketCap) return hipErrorInvalidValue;
+    bucket_sort_kernel<<<1, 256, 0, stream>>>(ev, n, k, nullptr, nullptr, nullptr, nullptr, cut, sorted, scratch);
+    return hipGetLastError();
+  }
+  const int buckets = 1 << bucket_bits;
+  const int shift = vmax(0, k.bits() - bucket_bits);
+  uint32_t *counts = words, *base = words + buckets, *cursor = words + 2 * buckets;
+  fill_counts_kernel<<<(buckets + 255) / 256, 256, 0, stream>>>(counts, buckets);
+  bucket_count_kernel<<<grid(n), 256, 0, stream>>>(ev, n, k, shift, static_cast<uint32_t>(buckets), counts);
+  bucket_scan_kernel<<<1, 1024, 0, stream>>>(counts, buckets, base, cursor, scratch);
+  bucket_fill_kernel<<<grid(n), 256, 0, stream>>>(ev, n, k, shift, static_cast<uint32_t>(buckets), cursor, keys, perm);
+  bucket_sort_kernel<<<buckets, 256, 0, stream>>>(ev, n, k, counts, base, keys, perm, cut, sorted, scratch);
+  return hipGetLastError();
+}
+
+hipError_t launch_out_reset_ready(unsigned long long* scratch, hipStream_t stream) {
+  fill_counts_kernel<<<1, 64, 0, stream>>>(reinterpret_cast<uint32_t*>(scratch + kOutReady), 2);
   return hipGetLastError();
 }
 

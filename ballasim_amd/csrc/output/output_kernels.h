@@ -7,15 +7,32 @@
 
 namespace bsx {
 
-// scratch: [0] kept count, [1..4] min/max of t_cross and t_reported (biased), [5] released count.
-inline constexpr int kOutScratch = 8;
+// scratch words: the kept new events, the extremes of t_reported and of the lag t_cross - t_reported over the
+// held and new events (biased to unsigned order), the released events, the largest bucket.
+enum OutScratch : int { kOutKept, kOutRepMin, kOutRepMax, kOutLagMin, kOutLagMax, kOutReady, kOutMostBucket, kOutScratch };
 
-// Appends the kept raw events as OutEventDev at out (count in scratch[0], which the caller zeroes).
+// The integer whose order is the output order: t_reported - rep_min, x, y and the lag t_cross - t_reported less
+// lag_min, from the leading bits down.
+struct OrderKey {
+  int64_t rep_min, lag_min;
+  int32_t rep_bits, x_bits, y_bits, lag_bits;
+  BSX_HD int bits() const { return rep_bits + x_bits + y_bits + lag_bits; }
+};
+inline constexpr int kMaxBucketBits = 14;
+
+// Resets scratch, appends the kept raw events as OutEventDev at held[n_held ..] and folds the extremes.
 hipError_t launch_out_build(const RawEventDev* raw, size_t n, uint32_t width, const Readout& r, bool crop,
-                            const CropBox& box, OutEventDev* out, unsigned long long* scratch, hipStream_t stream);
-// min/max of t_cross and t_reported over ev[0 .. n_held + scratch[0]) (grid over n_max).
-hipError_t launch_out_minmax(const OutEventDev* ev, size_t n_held, size_t n_max, unsigned long long* scratch,
-                             hipStream_t stream);
+                            const CropBox& box, OutEventDev* held, size_t n_held, unsigned long long* scratch,
+                            hipStream_t stream);
+// The bucket sort of ev[0 .. n) into sorted by a key of at most 64 bits, the events reported before cut counted:
+// 2^bucket_bits buckets (out_bucket_bits(n); 0: n events fit one block), words holds 3 << bucket_bits. Complete
+// when the largest bucket (scratch) is at most out_bucket_cap().
+int out_bucket_bits(size_t n);
+size_t out_bucket_cap();
+hipError_t launch_out_buckets(const OutEventDev* ev, size_t n, const OrderKey& k, int bucket_bits, int64_t cut,
+                              uint32_t* words, uint64_t* keys, uint32_t* perm, OutEventDev* sorted,
+                              unsigned long long* scratch, hipStream_t stream);
+hipError_t launch_out_reset_ready(unsigned long long* scratch, hipStream_t stream);
 // keys[i] of pass (0: t_cross - tc_min, 1: (x << y_bits) | y, 2: t_reported - tr_min) of ev[perm[i]] (perm
 // null: identity, perm_init filled with it).
 hipError_t launch_out_keys(const OutEventDev* ev, const uint32_t* perm, uint32_t* perm_init, size_t n, int pass,
@@ -24,7 +41,7 @@ hipError_t launch_out_keys(const OutEventDev* ev, const uint32_t* perm, uint32_t
 // perm_out, and keys / perm are overwritten.
 hipError_t launch_out_sort(uint64_t* keys, uint64_t* keys_out, uint32_t* perm, uint32_t* perm_out, size_t n, int bits,
                            DeviceBuffer& temp, hipStream_t stream);
-// sorted[i] = ev[perm[i]], counting those reported before cut into scratch[5].
+// sorted[i] = ev[perm[i]], counting those reported before cut into scratch.
 hipError_t launch_out_gather(const OutEventDev* ev, const uint32_t* perm, size_t n, int64_t cut, OutEventDev* sorted,
                              unsigned long long* scratch, hipStream_t stream);
 // The C4 columns of ev[0 .. n).

@@ -18,10 +18,11 @@ class Crop(C.Structure):
     _fields_ = [("x0", C.c_int32), ("y0", C.c_int32), ("x1", C.c_int32), ("y1", C.c_int32)]
 
 
-class OutputEvents(C.Structure):
-    _fields_ = [("count", C.c_size_t), ("x", C.c_void_p), ("y", C.c_void_p), ("p", C.c_void_p), ("t", C.c_void_p),
+class OutputColumns(C.Structure):
+    """Host arrays the released events' columns are fetched into, in the order of _COLUMNS."""
+    _fields_ = [("x", C.c_void_p), ("y", C.c_void_p), ("p", C.c_void_p), ("t", C.c_void_p),
                 ("t_ns_rem", C.c_void_p), ("t_reported_ns", C.c_void_p), ("t_cross_ns", C.c_void_p),
-                ("label", C.c_void_p), ("flags", C.c_void_p), ("held", C.c_size_t)]
+                ("label", C.c_void_p), ("flags", C.c_void_p)]
 
 
 _COLUMNS = (("x", np.uint16), ("y", np.uint16), ("p", np.uint8), ("t", np.int64), ("t_ns_rem", np.uint16),
@@ -53,27 +54,28 @@ class OutputStage:
         except Exception:
             pass
 
-    def _columns(self, out):
-        self.held = out.held
-        res = {}
-        for name, dt in _COLUMNS:
-            a = np.empty(out.count, dt)
-            if out.count:
-                C.memmove(a.ctypes.data, getattr(out, name), a.nbytes)
-            res[name] = a
+    def _columns(self, count, stream):
+        """The released events' columns, fetched into arrays of their own."""
+        res = {name: np.empty(count, dt) for name, dt in _COLUMNS}
+        if count:
+            dst = OutputColumns(*[a.ctypes.data for a in res.values()])
+            _abi.check(self._lib.bsx_output_fetch(self._h, _stream(stream), C.byref(dst)))
         return res
 
     def window(self, events, t_w, stream=0):
         """events: (data_ptr, count) of a window's raw device events; returns the released columns."""
         ev = _abi.DeviceEvents(*events)
-        out = OutputEvents()
-        _abi.check(self._lib.bsx_output_window(self._h, C.byref(ev), int(t_w), _stream(stream), C.byref(out)))
-        return self._columns(out)
+        n, held = C.c_size_t(), C.c_size_t()
+        _abi.check(self._lib.bsx_output_window_count(self._h, C.byref(ev), int(t_w), _stream(stream), C.byref(n),
+                                                     C.byref(held)))
+        self.held = held.value
+        return self._columns(n.value, stream)
 
     def flush(self, stream=0):
-        out = OutputEvents()
-        _abi.check(self._lib.bsx_output_flush(self._h, _stream(stream), C.byref(out)))
-        return self._columns(out)
+        n = C.c_size_t()
+        _abi.check(self._lib.bsx_output_flush_count(self._h, _stream(stream), C.byref(n)))
+        self.held = 0
+        return self._columns(n.value, stream)
 
 
 STREAM_EVENT = np.dtype([("t_reported_ns", np.int64), ("x", np.uint16), ("y", np.uint16), ("p", np.uint8),

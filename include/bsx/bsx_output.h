@@ -54,6 +54,24 @@ int bsx_output_window(bsx_output* o, const bsx_device_events* events, int64_t t_
 /* Every held event, in output order (the end of a run). */
 int bsx_output_flush(bsx_output* o, void* stream, bsx_output_events* out);
 
+/* The same two calls with the released events left on the device, and their columns fetched into the caller's own
+ * host arrays (each with room for *released events) before the stage's next call. */
+typedef struct bsx_output_columns {
+  uint16_t* x;
+  uint16_t* y;
+  uint8_t* p;
+  int64_t* t;
+  uint16_t* t_ns_rem;
+  int64_t* t_reported_ns;
+  int64_t* t_cross_ns;
+  uint8_t* label;
+  uint16_t* flags;
+} bsx_output_columns;
+int bsx_output_window_count(bsx_output* o, const bsx_device_events* events, int64_t t_w, void* stream, size_t* released,
+                            size_t* held);
+int bsx_output_flush_count(bsx_output* o, void* stream, size_t* released);
+int bsx_output_fetch(bsx_output* o, void* stream, const bsx_output_columns* dst);
+
 /* ---- Event stream: released events to the host in double-buffered pinned chunks ----
  *
  * No counterpart in the reference, whose engine hands each window's events to the writer on the host

@@ -135,3 +135,56 @@ def test_output_order_of_millions_of_events():
     want = oracle.flush()
     for k_got, k_want in (("x", "x"), ("y", "y"), ("t_reported_ns", "t_reported"), ("t_cross_ns", "t_cross")):
         assert np.array_equal(got[k_got], want[k_want]), k_got
+
+
+RAW_EVENT = np.dtype([("pixel", np.uint32), ("polarity", np.uint8), ("label", np.uint8), ("flags", np.uint16),
+                      ("t_cross", np.int64), ("ds", np.float32), ("dn", np.float32), ("dl", np.float32),
+                      ("l_first", np.float32)])
+
+
+# One block's sort and its edges, the first sizes that are bucketed, a quantum so coarse that buckets overflow
+# (the digit sort takes over), a drift that gives neighbouring times one report, keys of more than 64 bits, and a
+# column copy of several chunks.
+@pytest.mark.parametrize("n,size,readout,span", [
+    (1, (3, 2), {}, W), (2, (3, 2), {}, 3), (63, (40, 24), {}, W), (65, (40, 24), dict(readout_quantum_s=1e-6), W),
+    (2048, (640, 480), dict(readout_quantum_s=2e-5), W), (2049, (640, 480), {}, W),
+    (30000, (2048, 1536), dict(readout_quantum_s=5e-3), W), (30000, (64, 48), dict(readout_quantum_s=0.0,
+     clock_drift_ppm=-4000.0), 60000), (5000, (65535, 3), dict(readout_quantum_s=1.0), 1 << 40),
+    (300001, (1280, 720), dict(readout_quantum_s=1e-6, clock_drift_ppm=35.0), W)])
+def test_output_order_of_any_size(n, size, readout, span):
+    import torch
+
+    import ballasim_amd as bsx
+    from ballasim_amd.output import OutputStage
+    p = bsx.preset("prophesee_gen3")
+    p.photoreceptor = "instantaneous"
+    p.noise = False
+    for k, v in readout.items():
+        setattr(p, k, v)
+    p.readout_delay_s = max(p.readout_delay_s, p.readout_quantum_s)
+    w, h = size
+    m = bsx.SensorModel(p, w, h, 3, ["constant"], 0, device="cuda")
+    rd = dict(quantum=round(p.readout_quantum_s * 1e9), delay=round(p.readout_delay_s * 1e9),
+              phase=int(m._info().readout_phase_ns), offset=int(p.clock_offset_ns), drift_ppm=float(p.clock_drift_ppm))
+    rng = np.random.default_rng(n)
+    ev = np.zeros(n, RAW_EVENT)
+    ev["pixel"] = rng.integers(0, w * h, n)
+    ev["polarity"] = rng.integers(0, 2, n)
+    ev["label"] = rng.integers(0, 4, n)
+    ev["flags"] = rng.integers(0, 1 << 14, n)
+    ev["t_cross"] = 1 + rng.permutation(np.arange(n) * (span - 1) // n)  # (distinct, or distinct per pixel below)
+    keep = np.unique(ev[["pixel", "t_cross"]], return_index=True)[1]
+    ev = ev[np.sort(keep)]
+    stage = OutputStage(m)
+    oracle = Q.OutputOracle(w, h, rd)
+    dev = torch.from_numpy(ev.view(np.uint8).reshape(len(ev), 32)).cuda()
+    torch.cuda.synchronize()
+    raw = np.zeros(len(ev), O.EVENT_DTYPE)
+    for f in ("pixel", "polarity", "label", "flags", "t_cross"):
+        raw[f] = ev[f]
+    for got, want in ((stage.window((dev.data_ptr(), len(ev)), 0), oracle.window(raw, 0)),
+                      (stage.flush(), oracle.flush())):
+        for a, b in (("x", "x"), ("y", "y"), ("p", "p"), ("t", "t"), ("t_ns_rem", "t_ns_rem"),
+                     ("t_reported_ns", "t_reported"), ("t_cross_ns", "t_cross"), ("label", "label"), ("flags", "flags")):
+            assert np.array_equal(got[a], want[b]), a
+    assert stage.held == 0
