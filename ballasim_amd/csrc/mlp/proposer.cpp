@@ -53,19 +53,19 @@ void Proposer::get_params(float* w) const {
 double Proposer::gradients(const float* x, const float* t, int64_t n, float* grad, hipStream_t stream) {
   using namespace mlp;
   if (n <= 0) throw std::invalid_argument("Proposer.gradients: need at least one row");
-  const int64_t groups = (n + 63) / 64;
-  partial_.ensure(static_cast<size_t>(groups) * kParams * 4);
-  loss_.ensure(static_cast<size_t>(groups) * 4);
+  const int partials = gradient_partials(n);
+  partial_.ensure(static_cast<size_t>(partials) * kParams * 4);
+  loss_.ensure(static_cast<size_t>(partials) * 4);
   hip_check(launch_gradients(wb_.as<const uint16_t>(), w_.as<const float>(), x, t, n, n, partial_.as<float>(),
                              loss_.as<float>(), stream),
             "gradients");
   const Adam none{0.0f, 0.9f, 0.999f, 1e-8f, 1};
-  hip_check(launch_adam(partial_.as<const float>(), static_cast<int>(groups), grad_.as<float>(), w_.as<float>(),
-                        m_.as<float>(), v_.as<float>(), wb_.as<uint16_t>(), none, stream),
+  hip_check(launch_adam(partial_.as<const float>(), partials, grad_.as<float>(), w_.as<float>(), m_.as<float>(),
+                        v_.as<float>(), wb_.as<uint16_t>(), none, stream),
             "reduce gradients");
-  std::vector<float> lp(groups);
+  std::vector<float> lp(partials);
   hip_check(hipMemcpyAsync(grad, grad_.get(), kParams * 4, hipMemcpyDeviceToHost, stream), "download gradient");
-  hip_check(hipMemcpyAsync(lp.data(), loss_.get(), groups * 4, hipMemcpyDeviceToHost, stream), "download loss");
+  hip_check(hipMemcpyAsync(lp.data(), loss_.get(), lp.size() * 4, hipMemcpyDeviceToHost, stream), "download loss");
   hip_check(hipStreamSynchronize(stream), "gradients");
   double s = 0.0;
   for (const float v : lp) s += v;
@@ -78,23 +78,25 @@ double Proposer::train(const float* x, const float* t, int64_t n, int batch, int
     throw std::invalid_argument("Proposer.train: need rows, a batch that is a positive multiple of 64, epochs >= 1 "
                                 "and lr > 0");
   }
-  const int64_t groups = (n + 63) / 64;
-  partial_.ensure(static_cast<size_t>(batch / 64) * kParams * 4);
-  loss_.ensure(static_cast<size_t>(groups) * 4);
+  const int per_batch = gradient_partials(std::min<int64_t>(batch, n));
+  const int64_t steps = (n + batch - 1) / batch;
+  partial_.ensure(static_cast<size_t>(per_batch) * kParams * 4);
+  const size_t losses = static_cast<size_t>(steps - 1) * per_batch + gradient_partials(n - (steps - 1) * batch);
+  loss_.ensure(losses * 4);
   for (int e = 0; e < epochs; ++e) {
-    for (int64_t s = 0; s < n; s += batch) {
-      const int64_t nb = std::min<int64_t>(batch, n - s);
+    for (int64_t k = 0; k < steps; ++k) {
+      const int64_t s = k * batch, nb = std::min<int64_t>(batch, n - s);
       hip_check(launch_gradients(wb_.as<const uint16_t>(), w_.as<const float>(), x + s * kIn, t + s, nb, nb,
-                                 partial_.as<float>(), loss_.as<float>() + s / 64, stream),
+                                 partial_.as<float>(), loss_.as<float>() + k * per_batch, stream),
                 "gradients");
       const Adam a{lr, 0.9f, 0.999f, 1e-8f, static_cast<int32_t>(++step_)};
-      hip_check(launch_adam(partial_.as<const float>(), static_cast<int>((nb + 63) / 64), grad_.as<float>(),
-                            w_.as<float>(), m_.as<float>(), v_.as<float>(), wb_.as<uint16_t>(), a, stream),
+      hip_check(launch_adam(partial_.as<const float>(), gradient_partials(nb), grad_.as<float>(), w_.as<float>(),
+                            m_.as<float>(), v_.as<float>(), wb_.as<uint16_t>(), a, stream),
                 "adam");
     }
   }
-  std::vector<float> lp(groups);
-  hip_check(hipMemcpyAsync(lp.data(), loss_.get(), groups * 4, hipMemcpyDeviceToHost, stream), "download loss");
+  std::vector<float> lp(losses);
+  hip_check(hipMemcpyAsync(lp.data(), loss_.get(), lp.size() * 4, hipMemcpyDeviceToHost, stream), "download loss");
   hip_check(hipStreamSynchronize(stream), "train");
   double s = 0.0;
   for (const float v : lp) s += v;

@@ -97,3 +97,35 @@ def test_training_fits_a_smooth_target():
     loss = p.train(xd, td, batch=1024, epochs=8, lr=3e-3)
     _, l1 = p.gradients(xd, td)
     assert l1 < 0.05 * l0, (l0, loss, l1)
+
+
+# Row counts around a wave's 32 and 64 rows and a block's 256, more than one pass of every block (512 x 256 rows),
+# and rows that start off a 16-byte boundary (the scalar loads).
+@pytest.mark.parametrize("n,shift", [(1, 0), (31, 1), (33, 0), (255, 2), (257, 0), (131072 + 300, 0), (5000, 3)])
+def test_rows_of_any_count_and_alignment(n, shift):
+    import torch
+
+    from ballasim_amd.learned import Proposer
+    w, rng = _random_net(n)
+    p = Proposer(7)
+    p.params = w
+    x = rng.normal(0, 1, (n, 12)).astype(np.float32)
+    t = rng.normal(0, 1, n).astype(np.float32)
+    flat = torch.empty(n * 12 + 4, dtype=torch.float32, device="cuda")
+    xd = flat[shift:shift + n * 12].view(n, 12)
+    xd.copy_(torch.from_numpy(x))
+    y = torch.full((n + 1,), 7.0, device="cuda")
+    p.predict(xd, y)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    want, _ = M.forward(w, x)
+    assert got[n] == 7.0  # nothing past the rows
+    # (the bounds of test_forward_matches_oracle: the activations' rounding to bf16 may go the other way)
+    np.testing.assert_allclose(got[:n], want, rtol=1e-2, atol=2e-2)
+    assert np.median(np.abs(got[:n] - want)) < 1e-3
+    g, loss = p.gradients(xd, _dev(t))
+    gw, lw = M.gradients(w, x, t)
+    assert abs(loss - lw) <= 1e-3 * (1 + lw)
+    for a, b in ((M.OFF_W1, M.OFF_B1), (M.OFF_B1, M.OFF_W2), (M.OFF_W2, M.OFF_B2), (M.OFF_B2, M.OFF_W3),
+                 (M.OFF_W3, M.OFF_B3), (M.OFF_B3, M.N_PARAMS)):
+        assert np.linalg.norm(g[a:b] - gw[a:b]) <= 2e-2 * (np.linalg.norm(gw[a:b]) + 1e-6), (a, b)
