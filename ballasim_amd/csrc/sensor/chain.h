@@ -55,7 +55,7 @@ class LaunchChain {
   void capture();
   void drop_graph();
 
-  WalkTuning tu_{256, 8, 8, 0};
+  WalkTuning tu_{256, 4, 4, 0};
   bool graph_on_ = true;
   ChainStats stats_{};
 

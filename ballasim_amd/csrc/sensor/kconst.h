@@ -163,10 +163,11 @@ struct CallDev {
   int64_t n_runs;
 };
 
-// The walk's launch shape, chosen by the autotuner: threads per block, segments a walking lane does
-// before the wave looks again, waiting lanes that start a joint search, groups a wave takes per grab
-// of the persistent queue (0: one group per wave, no queue), and the head of the heavy-first order
-// walked in groups of fewer than 64 pixels.
+// The walk's launch shape, chosen by the autotuner: threads per block and, for the instantaneous walk,
+// segments a walking lane does before the wave looks again, waiting lanes that start a joint search and idle
+// lanes that take pixels from the queue together (0: 48). The walk with in-path noise takes its pixels 64 at a
+// time: chunk is the groups a wave takes per grab of the queue (0: one group per wave, no queue), and the head of
+// the heavy-first order may be walked in groups of fewer than 64 pixels.
 struct WalkTuning {
   int32_t block;
   int32_t walk_budget;

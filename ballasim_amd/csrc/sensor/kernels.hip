@@ -641,119 +641,203 @@ __device__ __forceinline__ void camera_add(const CameraDev* cams, int cam_index,
   }
 }
 
-// One 64-pixel group of the walk: lane i of the launch's pixel order takes pixel order[i] (of its
-// camera), walks it to t_end and writes its state. The wave's lanes walk their pixels; a lane that
-// reaches an exact search waits until search_batch lanes wait (or none walks), and then all waiting
-// lanes search together, so the searches of different pixels run side by side.
+// The pixels a wave's lanes take in turn: positions of the launch's heavy-first order. With a queue the grid
+// is resident and persistent: the first pixels are dealt out one per wave, wave after wave, so that the
+// heaviest lie in different waves, and later ones are taken from the queue. Without one each lane takes the
+// pixel of its place.
+struct LaneFeed {
+  uint32_t n_total, wave, n_waves, dealt;
+  unsigned int* queue;
+  bool begun = false, exhausted = false;  // (uniform over the wave)
+
+  __device__ __forceinline__ LaneFeed(uint32_t n, unsigned int* q) : n_total(n), queue(q) {
+    n_waves = gridDim.x * (blockDim.x / 64);
+    wave = (blockIdx.x * blockDim.x + threadIdx.x) / 64;
+    const uint32_t each = (n + n_waves - 1) / n_waves;
+    dealt = (each < 64 ? each : 64) * n_waves;
+  }
+
+  // Positions for the `wants` lanes (past n_total: none). Called by every lane of the wave.
+  __device__ __forceinline__ uint32_t take(bool wants) {
+    const uint32_t lane = __lane_id();
+    if (exhausted) return 0xffffffffu;
+    if (queue == nullptr) {
+      exhausted = true;
+      return wave * 64 + lane;
+    }
+    if (!begun) {
+      begun = true;
+      exhausted = dealt >= n_total;
+      return lane * n_waves < dealt ? lane * n_waves + wave : 0xffffffffu;
+    }
+    const unsigned long long waiting = __ballot(wants);
+    uint32_t first = 0;
+    if (lane == 0) first = atomicAdd(queue, static_cast<unsigned int>(__popcll(waiting)));
+    first = dealt + __shfl(first, 0);
+    exhausted = first + static_cast<uint32_t>(__popcll(waiting)) >= n_total;
+    return first + static_cast<uint32_t>(__popcll(waiting & ((1ull << lane) - 1ull)));
+  }
+};
+
+// An instantaneous lane's constants of its camera.
 template <int kMaxG>
-__device__ __forceinline__ void instant_group(const CameraDev* cams, int n_cams, uint32_t n_total,
-                                              const uint32_t* order, uint32_t i, const WalkTuning& tu,
-                                              int64_t t_end, uint32_t* stacks) {
-  InstantLane<kMaxG> L;
-  L.n_substeps = L.n_pieces = L.n_leaves = 0;
-  int ci = -1;
-  const CameraDev* cam = cams;
-  int p = 0;
-  if (i < n_total) {
-    const uint32_t g = order != nullptr ? order[i] : i;
-    ci = camera_of(cams, n_cams, g);
-    cam = cams + ci;
-    p = static_cast<int>(g - cam->base);
-  }
-  RigSink sink{cam, ci};
+__device__ __forceinline__ void instant_constants(InstantLane<kMaxG>& L, const CameraDev* cam) {
   const KConst& kc = cam->kc;
-  if (ci >= 0) {
-    const MapsDev& mp = cam->mp;
-    const StateDev& in = cam->in;
-    const RunsDev& runs = cam->runs;
-    L.pixel = static_cast<uint32_t>(p);
-    L.theta_on = mp.theta_on[p];
-    L.theta_off = mp.theta_off[p];
-    L.leak = mp.leak[p];
-    L.dark = mp.dark[p];
-    L.scale = mp.scale[p];
-    L.irr_max = kc.irr_max;
-    L.eps_ci = kc.eps_ci;
-    L.label_cut = kc.label_cut;
-    L.refractory_ns = kc.refractory_ns;
-    L.G = kc.groups;
-    L.ideal_reset = kc.ideal_reset != 0;
-    L.hot = mp.hot[p] != 0;
-    const int32_t row = runs.row_of != nullptr ? runs.row_of[p] : -1;
-    int loud_start = 0;
-    if (row >= 0) {
-      const int64_t start = runs.row_start[row];
-      L.ts = runs.t + start;
-      L.irr = runs.irr + start * kc.groups;
-      L.n = runs.row_count[row];
-      if (cam->first_loud != nullptr) loud_start = vmin(cam->first_loud[row], L.n);
-      if (cam->screen_blocks != nullptr) {
-        L.qb = cam->screen_blocks;
-        L.q_base = cam->pos[row];
-      }
-    } else {
-      L.ts = nullptr;
-      L.irr = nullptr;
-      L.n = 0;
+  L.irr_max = kc.irr_max;
+  L.eps_ci = kc.eps_ci;
+  L.label_cut = kc.label_cut;
+  L.refractory_ns = kc.refractory_ns;
+  L.G = kc.groups;
+  L.ideal_reset = kc.ideal_reset != 0;
+  L.t_state = cam->t_state;
+  L.shot_rate = kc.shot_rate_hz;
+  L.seed = kc.seed;
+  L.camera = kc.camera;
+}
+
+// An instantaneous lane's pixel p of camera cam: its maps, its run from its first loud segment and its state.
+template <int kMaxG>
+__device__ __forceinline__ void instant_setup(InstantLane<kMaxG>& L, const CameraDev* cam, int p, int64_t t_end) {
+  const KConst& kc = cam->kc;
+  const MapsDev& mp = cam->mp;
+  const StateDev& in = cam->in;
+  const RunsDev& runs = cam->runs;
+  L.pixel = static_cast<uint32_t>(p);
+  L.theta_on = mp.theta_on[p];
+  L.theta_off = mp.theta_off[p];
+  L.leak = mp.leak[p];
+  L.dark = mp.dark[p];
+  L.scale = mp.scale[p];
+  L.hot = mp.hot[p] != 0;
+  const int32_t row = runs.row_of != nullptr ? runs.row_of[p] : -1;
+  int loud_start = 0;
+  L.qb = nullptr;
+  if (row >= 0) {
+    const int64_t start = runs.row_start[row];
+    L.ts = runs.t + start;
+    L.irr = runs.irr + start * kc.groups;
+    L.n = runs.row_count[row];
+    if (cam->first_loud != nullptr) loud_start = vmin(cam->first_loud[row], L.n);
+    if (cam->screen_blocks != nullptr) {
+      L.qb = cam->screen_blocks;
+      L.q_base = cam->pos[row];
     }
-    L.t_state = cam->t_state;
-    L.skip = L.n > 0 && L.ts[0] == L.t_state ? 1 : 0;
-    for (int g = 0; g < kMaxG; ++g)
-      if (g < kc.groups) L.held[g] = in.held[static_cast<int64_t>(g) * kc.n_pixels + p];
-    L.i_scale = in.i_scale[p];
-    L.s3_ref = in.s3_ref[p];
-    L.n3_ref = in.n3_ref[p];
-    L.dr_ref = in.dr_ref[p];
-    L.t_ref = in.t_ref[p];
-    L.blind_until = in.blind_until[p];
-    L.t_search = in.t_search[p];
-    L.flags = in.flags[p];
-    L.shot_rate = kc.shot_rate_hz;
-    L.seed = kc.seed;
-    L.camera = kc.camera;
-    L.shot_next = in.shot_next[p];
-    L.shot_index = in.shot_index[p];
-    L.begin(t_end, loud_start);
+  } else {
+    L.ts = nullptr;
+    L.irr = nullptr;
+    L.n = 0;
   }
-  int mode = ci >= 0 ? L.walk(sink, tu.walk_budget) : InstantLane<kMaxG>::kDone;
-  while (true) {
-    const unsigned long long searching = __ballot(mode == InstantLane<kMaxG>::kSearch);
-    const unsigned long long walking = __ballot(mode == InstantLane<kMaxG>::kWalk);
-    if ((searching | walking) == 0) break;
-    if (searching != 0 && (walking == 0 || __popcll(searching) >= tu.search_batch)) {
-      if (mode == InstantLane<kMaxG>::kSearch) {
-        L.search_step(sink, stacks, blockDim.x);
-        mode = InstantLane<kMaxG>::kWalk;
-      }
-    } else if (mode == InstantLane<kMaxG>::kWalk) {
-      mode = L.walk(sink, tu.walk_budget);
-    }
-  }
-  if (ci >= 0) {
-    const StateDev& in = cam->in;
-    const StateDev& out = cam->out;
-    L.end();
-    for (int g = 0; g < kMaxG; ++g)
-      if (g < kc.groups) out.held[static_cast<int64_t>(g) * kc.n_pixels + p] = L.held[g];
-    out.z[p] = in.z[p];
-    out.x1[p] = in.x1[p];
-    out.s2[p] = in.s2[p];
-    out.s3[p] = in.s3[p];
-    out.tv[p] = in.tv[p];
-    out.i_scale[p] = L.i_scale;
-    out.s3_ref[p] = L.s3_ref;
-    out.n3_ref[p] = L.n3_ref;
-    out.dr_ref[p] = L.dr_ref;
-    out.t_ref[p] = L.t_ref;
-    out.blind_until[p] = L.blind_until;
-    out.t_search[p] = L.t_search;
-    out.flags[p] = static_cast<uint16_t>(L.flags);
-    out.shot_next[p] = L.shot_next;
-    out.shot_index[p] = L.shot_index;
-  }
+  L.skip = L.n > 0 && L.ts[0] == L.t_state ? 1 : 0;
+  for (int g = 0; g < kMaxG; ++g)
+    if (g < kc.groups) L.held[g] = in.held[static_cast<int64_t>(g) * kc.n_pixels + p];
+  L.i_scale = in.i_scale[p];
+  L.s3_ref = in.s3_ref[p];
+  L.n3_ref = in.n3_ref[p];
+  L.dr_ref = in.dr_ref[p];
+  L.t_ref = in.t_ref[p];
+  L.blind_until = in.blind_until[p];
+  L.t_search = in.t_search[p];
+  L.flags = in.flags[p];
+  L.shot_next = in.shot_next[p];
+  L.shot_index = in.shot_index[p];
+  L.scr_valid = false;
+  L.st_I = -1.0f;
+  L.begin(t_end, loud_start);
+}
+
+// A finished instantaneous lane's end() and its pixel's new state.
+template <int kMaxG>
+__device__ __forceinline__ void instant_store(InstantLane<kMaxG>& L, const CameraDev* cam, int p) {
+  const KConst& kc = cam->kc;
+  const StateDev& in = cam->in;
+  const StateDev& out = cam->out;
+  L.end();
+  for (int g = 0; g < kMaxG; ++g)
+    if (g < kc.groups) out.held[static_cast<int64_t>(g) * kc.n_pixels + p] = L.held[g];
+  out.z[p] = in.z[p];
+  out.x1[p] = in.x1[p];
+  out.s2[p] = in.s2[p];
+  out.s3[p] = in.s3[p];
+  out.tv[p] = in.tv[p];
+  out.i_scale[p] = L.i_scale;
+  out.s3_ref[p] = L.s3_ref;
+  out.n3_ref[p] = L.n3_ref;
+  out.dr_ref[p] = L.dr_ref;
+  out.t_ref[p] = L.t_ref;
+  out.blind_until[p] = L.blind_until;
+  out.t_search[p] = L.t_search;
+  out.flags[p] = static_cast<uint16_t>(L.flags);
+  out.shot_next[p] = L.shot_next;
+  out.shot_index[p] = L.shot_index;
+}
+
+template <int kMaxG>
+__device__ __forceinline__ void instant_count(const CameraDev* cams, int ci, InstantLane<kMaxG>& L) {
   camera_add(cams, ci, 1 + kStSubsteps, L.n_substeps);
   camera_add(cams, ci, 1 + kStPieces, L.n_pieces);
   camera_add(cams, ci, 1 + kStLeaves, L.n_leaves);
+}
+
+// The instantaneous walk. The wave's lanes walk their pixels; a lane that reaches an exact search waits until
+// search_batch lanes wait (or none walks), and then all waiting lanes search together, so the searches of
+// different pixels run side by side. A lane whose pixel is done takes another (LaneFeed), `refill` lanes at a time.
+// Bound by the latency of the lanes' dependent steps: dealing the heaviest pixels one to a wave, where a wave of 64
+// of them set the walk's length, took a 1280x720 window's chain from 2.46 to 2.19 ms, a 2048x1536 window's from
+// 16.6 to 13.5 and a 64x48 call's from 0.36 to 0.23 (refill 8: 14.1 ms of 2048x1536, 16: 13.8, 48: 13.5, 64:
+// 14.2; walk_budget 1, 2, 4, 8: 14.8, 14.4, 13.5, 14.5; search_batch 2, 4, 16: 13.6, 13.5, 13.9).
+template <int kMaxG, bool kOne>
+__device__ __forceinline__ void instant_lanes(const CameraDev* cams, int n_cams, uint32_t n_total, const uint32_t* order,
+                                              unsigned int* queue, const WalkTuning& tu, int64_t t_end,
+                                              uint32_t* stacks) {
+  using Lane = InstantLane<kMaxG>;
+  constexpr int kIdle = -1, kOut = -2;  // waiting for a pixel (the last one not saved yet); none left
+  const int refill = tu.chunk > 0 ? tu.chunk : 48;  // idle lanes that take pixels together
+  LaneFeed feed(n_total, queue);
+  Lane L;
+  L.n_substeps = L.n_pieces = L.n_leaves = 0;
+  int mode = kIdle, ci = -1, p = 0;
+  if constexpr (kOne) instant_constants(L, cams);
+  while (true) {
+    if (mode == Lane::kDone) mode = kIdle;
+    const int idle = __popcll(__ballot(mode == kIdle)), searching = __popcll(__ballot(mode == Lane::kSearch)),
+              walking = __popcll(__ballot(mode == Lane::kWalk));
+    if (idle + searching + walking == 0) break;
+    if (idle > 0 && (searching + walking == 0 || feed.exhausted || idle >= refill)) {
+      // save the finished pixels and take new ones (a rig's counters are kept per pixel, as the next one's
+      // camera may be another)
+      const bool done = mode == kIdle && ci >= 0;
+      if (done) instant_store(L, kOne ? cams : cams + ci, p);
+      if constexpr (!kOne) {
+        instant_count(cams, done ? ci : -1, L);
+        if (done) L.n_substeps = L.n_pieces = L.n_leaves = 0;
+      }
+      const uint32_t i = feed.take(mode == kIdle);
+      if (mode == kIdle) {
+        ci = -1;
+        mode = kOut;
+        if (i < n_total) {
+          const uint32_t g = order != nullptr ? order[i] : i;
+          ci = kOne ? 0 : camera_of(cams, n_cams, g);
+          const CameraDev* cam = kOne ? cams : cams + ci;
+          p = static_cast<int>(g - cam->base);
+          if constexpr (!kOne) instant_constants(L, cam);
+          instant_setup(L, cam, p, t_end);
+          mode = Lane::kWalk;
+        }
+      }
+      continue;
+    }
+    RigSink sink{kOne ? cams : cams + ci, ci};
+    if (searching != 0 && (walking == 0 || searching >= tu.search_batch)) {
+      if (mode == Lane::kSearch) {
+        L.search_step(sink, stacks, blockDim.x);
+        mode = Lane::kWalk;
+      }
+    } else if (mode == Lane::kWalk) {
+      mode = L.walk(sink, tu.walk_budget);
+    }
+  }
+  if constexpr (kOne) instant_count(cams, 0, L);
 }
 
 // The walk's groups over n pixels of the heavy-first order: tu.head_groups groups of tu.head_lanes
@@ -796,18 +880,15 @@ __device__ __forceinline__ void walk_groups(uint32_t n_total, unsigned int* queu
 
 // Three waves per SIMD: the register allocation is held to 168 (a few bytes of scratch per lane
 // beyond it), which measured faster than 173 registers at two waves.
-template <int kMaxG>
-__global__ __launch_bounds__(kInstantBlock) __attribute__((amdgpu_waves_per_eu(3))) void instant_walk_kernel(const CameraDev* cams, int n_cams, uint32_t n_total,
-                                                                   const uint32_t* order, unsigned int* queue,
-                                                                   WalkTuning tu, const CallDev* call) {
+template <int kMaxG, bool kOne>
+__global__ __launch_bounds__(kInstantBlock) __attribute__((amdgpu_waves_per_eu(3))) void instant_walk_kernel(
+    const CameraDev* cams, int n_cams, uint32_t n_total, const uint32_t* order, unsigned int* queue, WalkTuning tu,
+    const CallDev* call) {
   if (call_refused(cams, n_cams)) return;
   // The lanes' bisection stacks, one column per lane (conflict-free: a level is a row of the block;
   // blockDim.x <= kInstantBlock by the launch bound).
   __shared__ uint32_t stacks[InstantLane<kMaxG>::kSearchDepth * kInstantBlock];
-  const int64_t t_end = call->t_end;
-  walk_groups(n_total, queue, tu, [&](uint32_t i) {
-    instant_group<kMaxG>(cams, n_cams, n_total, order, i, tu, t_end, stacks + threadIdx.x);
-  });
+  instant_lanes<kMaxG, kOne>(cams, n_cams, n_total, order, queue, tu, call->t_end, stacks + threadIdx.x);
 }
 
 // Phase A of the cascade, over every segment of every camera's runs (one thread per segment position).
@@ -966,44 +1047,6 @@ __device__ __forceinline__ void cascade_count(const CameraDev* cams, int ci, Cas
   camera_add(cams, ci, 1 + kStQuarantines, L.n_quarantines);
   camera_add(cams, ci, 1 + kStPieces, L.n_pieces);
 }
-
-// The pixels a wave's lanes take in turn: positions of the launch's heavy-first order. With a queue the grid
-// is resident and persistent: the first pixels are dealt out one per wave, wave after wave, so that the
-// heaviest lie in different waves, and later ones are taken from the queue. Without one each lane takes the
-// pixel of its place.
-struct LaneFeed {
-  uint32_t n_total, wave, n_waves, dealt;
-  unsigned int* queue;
-  bool begun = false, exhausted = false;  // (uniform over the wave)
-
-  __device__ __forceinline__ LaneFeed(uint32_t n, unsigned int* q) : n_total(n), queue(q) {
-    n_waves = gridDim.x * (blockDim.x / 64);
-    wave = (blockIdx.x * blockDim.x + threadIdx.x) / 64;
-    const uint32_t each = (n + n_waves - 1) / n_waves;
-    dealt = (each < 64 ? each : 64) * n_waves;
-  }
-
-  // Positions for the `wants` lanes (past n_total: none). Called by every lane of the wave.
-  __device__ __forceinline__ uint32_t take(bool wants) {
-    const uint32_t lane = __lane_id();
-    if (exhausted) return 0xffffffffu;
-    if (queue == nullptr) {
-      exhausted = true;
-      return wave * 64 + lane;
-    }
-    if (!begun) {
-      begun = true;
-      exhausted = dealt >= n_total;
-      return lane * n_waves < dealt ? lane * n_waves + wave : 0xffffffffu;
-    }
-    const unsigned long long waiting = __ballot(wants);
-    uint32_t first = 0;
-    if (lane == 0) first = atomicAdd(queue, static_cast<unsigned int>(__popcll(waiting)));
-    first = dealt + __shfl(first, 0);
-    exhausted = first + static_cast<uint32_t>(__popcll(waiting)) >= n_total;
-    return first + static_cast<uint32_t>(__popcll(waiting & ((1ull << lane) - 1ull)));
-  }
-};
 
 // The coefficients of the sub-step tries [0, h] with input Ia -> Ib that the lanes of `tries` are due
 // (cascade::try_coef, the same steps), worked out by the whole wave: four lanes share a try, sixteen tries at
@@ -1468,8 +1511,10 @@ int resident_blocks(int kind, int tier, int block) {
          reinterpret_cast<const void*>(cascade_walk_kernel<2, true>),
          reinterpret_cast<const void*>(cascade_walk_kernel<4, true>),
          reinterpret_cast<const void*>(cascade_walk_kernel<8, true>)},
-        {reinterpret_cast<const void*>(instant_walk_kernel<1>), reinterpret_cast<const void*>(instant_walk_kernel<2>),
-         reinterpret_cast<const void*>(instant_walk_kernel<4>), reinterpret_cast<const void*>(instant_walk_kernel<8>)},
+        {reinterpret_cast<const void*>(instant_walk_kernel<1, true>),
+         reinterpret_cast<const void*>(instant_walk_kernel<2, true>),
+         reinterpret_cast<const void*>(instant_walk_kernel<4, true>),
+         reinterpret_cast<const void*>(instant_walk_kernel<8, true>)},
         {reinterpret_cast<const void*>(noise_walk_kernel<1>), reinterpret_cast<const void*>(noise_walk_kernel<2>),
          reinterpret_cast<const void*>(noise_walk_kernel<4>), reinterpret_cast<const void*>(noise_walk_kernel<8>)}};
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernels[kind][tier], block, 0) != hipSuccess)
@@ -1521,7 +1566,7 @@ hipError_t launch_chain_prepare(const ChainArgs& a, hipStream_t stream) {
 int chain_walk_blocks(const ChainArgs& a) {
   const int block = a.tu.block;
   const unsigned full = static_cast<unsigned>((uint64_t{walk_group_count(a.n_total, a.tu)} * 64 + block - 1) / block);
-  const bool machines = !a.instant && !a.noise;  // the noise-free cascade's walk takes its pixels from the queue
+  const bool machines = !a.noise;  // walks whose lanes take their pixels from the queue
   if ((a.tu.chunk <= 0 && !machines) || a.queue == nullptr) return static_cast<int>(full);
   const int kind = a.instant ? 1 : a.noise ? 2 : 0;
   const unsigned resident = static_cast<unsigned>(resident_blocks(kind, group_tier(a.groups), block));
@@ -1535,35 +1580,25 @@ hipError_t launch_chain_walk(const ChainArgs& a, hipStream_t stream) {
   if (a.n_total == 0) return hipSuccess;
   const int block = a.tu.block, tier = group_tier(a.groups);
   const dim3 grid(static_cast<unsigned>(chain_walk_blocks(a)));
-#define BSX_WALK(K, G) K<G><<<grid, block, 0, stream>>>(a.cams, a.n_cams, a.n_total, a.perm, a.queue, a.tu, a.call)
-  if (a.instant) {
-    if (tier == 0) BSX_WALK(instant_walk_kernel, 1);
-    else if (tier == 1) BSX_WALK(instant_walk_kernel, 2);
-    else if (tier == 2) BSX_WALK(instant_walk_kernel, 4);
-    else BSX_WALK(instant_walk_kernel, 8);
-  } else if (a.noise) {
-    if (tier == 0) BSX_WALK(noise_walk_kernel, 1);
-    else if (tier == 1) BSX_WALK(noise_walk_kernel, 2);
-    else if (tier == 2) BSX_WALK(noise_walk_kernel, 4);
-    else BSX_WALK(noise_walk_kernel, 8);
-  } else {
-#define BSX_CASCADE(G)                                                                                           \
-  if (a.n_cams == 1)                                                                                             \
-    cascade_walk_kernel<G, true><<<grid, block, 0, stream>>>(a.cams, a.n_cams, a.n_total, a.perm, a.queue, a.tu, \
-                                                             a.call);                                            \
-  else                                                                                                           \
-    cascade_walk_kernel<G, false><<<grid, block, 0, stream>>>(a.cams, a.n_cams, a.n_total, a.perm, a.queue, a.tu, a.call)
-    if (tier == 0) {
-      BSX_CASCADE(1);
-    } else if (tier == 1) {
-      BSX_CASCADE(2);
-    } else if (tier == 2) {
-      BSX_CASCADE(4);
-    } else {
-      BSX_CASCADE(8);
-    }
-#undef BSX_CASCADE
-  }
+  // (a launch of one camera keeps the camera's constants in scalar registers)
+#define BSX_WALK(K, ...) K<__VA_ARGS__><<<grid, block, 0, stream>>>(a.cams, a.n_cams, a.n_total, a.perm, a.queue, a.tu, a.call)
+#define BSX_LANES(K, G)                       \
+  do {                                        \
+    if (a.n_cams == 1) BSX_WALK(K, G, true);  \
+    else BSX_WALK(K, G, false);               \
+  } while (0)
+#define BSX_TIERS(LAUNCH, K)       \
+  do {                             \
+    if (tier == 0) LAUNCH(K, 1);   \
+    else if (tier == 1) LAUNCH(K, 2); \
+    else if (tier == 2) LAUNCH(K, 4); \
+    else LAUNCH(K, 8);             \
+  } while (0)
+  if (a.instant) BSX_TIERS(BSX_LANES, instant_walk_kernel);
+  else if (a.noise) BSX_TIERS(BSX_WALK, noise_walk_kernel);
+  else BSX_TIERS(BSX_LANES, cascade_walk_kernel);
+#undef BSX_TIERS
+#undef BSX_LANES
 #undef BSX_WALK
   return hipGetLastError();
 }

@@ -46,7 +46,7 @@ int bsx_rig_advance_device(bsx_rig* rig, const bsx_device_runs* runs, int64_t t_
                            bsx_device_events* out);
 
 /* The walk's launch shape (the fields of bsx_launch_policy other than event_capacity; 0 in a field =
- * keep, queue_chunk -1 = no queue). A new shape re-captures the graph at the next call. */
+ * keep, queue_chunk -1 sets 0). A new shape re-captures the graph at the next call. */
 int bsx_rig_set_tuning(bsx_rig* rig, const bsx_launch_policy* tuning);
 int bsx_rig_get_tuning(bsx_rig* rig, bsx_launch_policy* out);
 /* Graph capture on (default) or off (kernel-by-kernel launches; same results). */

@@ -80,6 +80,36 @@ def test_instant_matches_oracle(case):
         assert ks[f] == ko[f], (f, ks[f], ko[f])
 
 
+# One pixel, one fewer and one more than a wave (and than the lanes that refill together), and more pixels than
+# the walk's resident lanes (256 CUs x 12 waves x 64), so that lanes take theirs from the queue; the launch
+# shapes that refill at every idle lane and at a whole wave of them.
+@pytest.mark.parametrize("W,H,frac", [(1, 1, 1.0), (47, 1, 1.0), (63, 1, 1.0), (65, 1, 0.9), (641, 331, 0.1)])
+@pytest.mark.parametrize("refill", [0, 1, 64])
+def test_lanes_take_pixels(W, H, frac, refill):
+    import ballasim_amd as bsx
+    rng = np.random.default_rng(W)
+    p = _params("physical_leak")
+    gpu = bsx.SensorModel(p, W, H, 5, ["constant"], 0, device="cuda")
+    if refill:
+        gpu.set_launch_policy(queue_chunk=refill)
+    ref = O.OracleModel(p.c, W, H, 5, 1, 0)
+    irr0 = np.exp(rng.normal(3, 1, size=(W * H, 1))).astype(np.float32)
+    gpu.init(0, irr0)
+    ref.init(0, irr0)
+    t = 0
+    for t1 in (2 ** 23, 2 ** 23 + 5 * 2 ** 20):
+        ids, ts, ir, offs = random_runs(rng, W * H, t, t1, frac=frac, max_n=40 if W * H < 100 else 8)
+        ev = gpu.advance(ids, ts, ir, t1, offsets=offs)
+        want, _ = ref.advance_runs(ids, ts, ir, offs, t1)
+        got = events_from_dict(ev, W)
+        i, a, b = first_difference(got, want)
+        assert len(got) == len(want) and i == len(got), f"first difference at {i}: gpu {a} oracle {b}"
+        t = t1
+    st = np.frombuffer(gpu.save_state()[56:], O.REF_STATE_DTYPE)
+    for f in ("s3_ref", "dr_ref", "i_scale", "t_ref", "t_search", "blind_until", "flags"):
+        assert np.array_equal(st[f], ref.states()[f]), f
+
+
 def test_padded_counts_and_unlisted_pixels():
     """The padded form with counts, a call with no listed pixels (held input, leak fires), and a
     zero-length call."""
