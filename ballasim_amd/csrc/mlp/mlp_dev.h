@@ -20,7 +20,6 @@ typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 inline constexpr int kS16 = 72;  // row stride (elements) of bf16 LDS matrices: 36 words, no bank aliasing
-inline constexpr int kS32 = 65;  // row stride of fp32 LDS matrices
 
 // fp32 -> bf16, round to nearest even (finite inputs).
 __host__ __device__ __forceinline__ uint16_t to_bf16(float f) {
@@ -40,11 +39,6 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 __device__ __forceinline__ float silu(float z) { return z / (1.0f + __expf(-z)); }
-// d silu / dz = s (1 + z (1 - s)), s = 1 / (1 + exp(-z)).
-__device__ __forceinline__ float silu_grad(float z) {
-  const float s = 1.0f / (1.0f + __expf(-z));
-  return s * (1.0f + z * (1.0f - s));
-}
 
 // acc += A . B over k = 0 .. K - 1 (K a multiple of 8) for the 32x32 tile whose A rows start at a and
 // B columns at b: A(m, k) = a[m * am + k * ak], B(k, n) = b[k * bk + n * bn] (bf16 in LDS). Called by
@@ -75,66 +69,116 @@ struct WeightsLds {
   float b3;
 };
 
-// Loads the weights into LDS (all threads of the block; a barrier follows).
-__device__ __forceinline__ void load_weights(WeightsLds& s, const uint16_t* wb, const float* w) {
-  for (int i = threadIdx.x; i < kInPad * kHid; i += blockDim.x) {
-    const int f = i / kHid, h = i % kHid;
-    s.w1[f * kS16 + h] = f < kIn ? wb[kOffW1 + f * kHid + h] : uint16_t{0};
-  }
-  for (int i = threadIdx.x; i < kHid * kHid; i += blockDim.x) s.w2[(i / kHid) * kS16 + i % kHid] = wb[kOffW2 + i];
-  for (int i = threadIdx.x; i < kHid; i += blockDim.x) {
-    s.b1[i] = w[kOffB1 + i];
-    s.b2[i] = w[kOffB2 + i];
-    s.w3[i] = from_bf16(wb[kOffW3 + i]);
-  }
-  if (threadIdx.x == 0) s.b3 = w[kOffB3];
-  __syncthreads();
-}
+// ---- One wave's 64 rows (the learned sampler) -------------------------------------------------------
+// The products run transposed, hidden units by rows: a lane's accumulators hold 32 units of one row, which,
+// rounded to bf16 four at a time, are the next product's B operand as they stand, so activations stay in
+// registers. (With the activations and two sets of pre-activations in LDS a wave took 64 KB, which left two waves
+// to a compute unit; it takes 15 KB here.) The sums over k and over the output's units run in the order of the
+// plain product, so that a sample time does not depend on the layout.
+inline constexpr int kS1 = 20, kS2 = 68;  // row strides (elements): 8-byte reads of 32 rows meet every bank once
 
-// One wave's activations in LDS: xs = the 64 input rows (bf16, columns 12 .. 31 zero), z1 and z2 the
-// pre-activations (fp32), h1 = bf16(silu(z1)).
-struct WaveLds {
-  uint16_t xs[kRowsPerWave * kS16];
-  float z1[kRowsPerWave * kS32];
-  float z2[kRowsPerWave * kS32];
-  uint16_t h1[kRowsPerWave * kS16];
+struct WaveWeights {
+  alignas(16) float b1[kHid];
+  alignas(16) float b2[kHid];
+  float w3[kHid];
+  float b3;
+  alignas(8) uint16_t w1[kHid * kS1];  // W1 by unit: 16 features (12 and four zeros)
+  alignas(8) uint16_t w2[kHid * kS2];  // W2 by output unit
+  alignas(8) uint16_t xs[kRowsPerWave * kS1];  // the rows' features, bf16
 };
 
-// Writes this lane's features as row (lane) of xs, then syncs the wave.
-__device__ __forceinline__ void put_features(WaveLds& s, const float* f) {
+typedef short bf16x4_lds __attribute__((ext_vector_type(4), may_alias));
+
+__device__ __forceinline__ short bf16_bits(float f) { return static_cast<short>(to_bf16(f)); }
+
+// Loads the weights (called by all 64 lanes; lane l takes unit l).
+__device__ __forceinline__ void load_weights(WaveWeights& s, const uint16_t* wb, const float* w) {
   const int l = threadIdx.x & 63;
-  for (int c = 0; c < kS16; ++c) s.xs[l * kS16 + c] = c < kIn ? to_bf16(f[c]) : uint16_t{0};
+  static_assert(kHid == 64 && kIn % 4 == 0 && kInPad == 16);
+#pragma unroll
+  for (int q = 0; q < kInPad / 4; ++q) {
+    bf16x4 v = {0, 0, 0, 0};
+    if (4 * q < kIn)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = static_cast<short>(wb[kOffW1 + (4 * q + i) * kHid + l]);
+    *reinterpret_cast<bf16x4_lds*>(s.w1 + l * kS1 + 4 * q) = v;
+  }
+#pragma unroll
+  for (int q = 0; q < kHid / 4; ++q) {
+    bf16x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = static_cast<short>(wb[kOffW2 + (4 * q + i) * kHid + l]);
+    *reinterpret_cast<bf16x4_lds*>(s.w2 + l * kS2 + 4 * q) = v;
+  }
+  s.b1[l] = w[kOffB1 + l];
+  s.b2[l] = w[kOffB2 + l];
+  s.w3[l] = from_bf16(wb[kOffW3 + l]);
+  if (l == 0) s.b3 = w[kOffB3];
   wave_sync();
 }
 
-// The forward pass of the wave's 64 rows (xs filled): z1, h1, z2 in LDS; returns this lane's row's y.
-__device__ __forceinline__ float wave_forward(const WeightsLds& w, WaveLds& s) {
-  for (int mt = 0; mt < 2; ++mt)
-    for (int nt = 0; nt < 2; ++nt) {
+// The network's output for each lane's features f[0 .. kIn - 1] (called by all 64 lanes).
+__device__ __forceinline__ float wave_forward(WaveWeights& s, const float* f) {
+  const int l = threadIdx.x & 63, r = l & 31, kq = (l >> 5) * 4;
+#pragma unroll
+  for (int q = 0; q < kInPad / 4; ++q) {
+    bf16x4 v = {0, 0, 0, 0};
+    if (4 * q < kIn)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = bf16_bits(f[4 * q + i]);
+    *reinterpret_cast<bf16x4_lds*>(s.xs + l * kS1 + 4 * q) = v;
+  }
+  wave_sync();
+  const auto operand = [](const uint16_t* p) { return *reinterpret_cast<const bf16x4_lds*>(p); };
+  uint32_t part[2][32];  // a unit's share of the output of row nt * 32 + l % 32: units acc_row, both tiles
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt) {
+    bf16x4 h1[8];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
       f32x16 acc = {};
-      mma_tile(acc, s.xs + mt * 32 * kS16, kS16, 1, w.w1 + nt * 32, kS16, 1, kInPad);
+#pragma unroll
+      for (int k0 = 0; k0 < kInPad; k0 += 8)
+        acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(operand(s.w1 + (mt * 32 + r) * kS1 + k0 + kq),
+                                                       operand(s.xs + (nt * 32 + r) * kS1 + k0 + kq), acc, 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        h1[mt * 4 + (j >> 2)][j & 3] = bf16_bits(silu(acc[j] + s.b1[mt * 32 + 8 * (j >> 2) + kq + (j & 3)]));
+    }
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      f32x16 acc = {};
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(operand(s.w2 + (mt * 32 + r) * kS2 + 8 * k + kq), h1[k], acc,
+                                                       0, 0, 0);
+#pragma unroll
       for (int j = 0; j < 16; ++j) {
-        const int r = mt * 32 + acc_row(j), c = nt * 32 + acc_col();
-        const float z = acc[j] + w.b1[c];
-        s.z1[r * kS32 + c] = z;
-        s.h1[r * kS16 + c] = to_bf16(silu(z));
+        const int u = mt * 32 + 8 * (j >> 2) + kq + (j & 3);
+        part[nt][mt * 16 + j] = __builtin_bit_cast(uint32_t, from_bf16(to_bf16(silu(acc[j] + s.b2[u]))) * s.w3[u]);
       }
     }
-  wave_sync();
-  for (int mt = 0; mt < 2; ++mt)
-    for (int nt = 0; nt < 2; ++nt) {
-      f32x16 acc = {};
-      mma_tile(acc, s.h1 + mt * 32 * kS16, kS16, 1, w.w2 + nt * 32, kS16, 1, kHid);
-      for (int j = 0; j < 16; ++j) {
-        const int r = mt * 32 + acc_row(j), c = nt * 32 + acc_col();
-        s.z2[r * kS32 + c] = acc[j] + w.b2[c];
-      }
-    }
-  wave_sync();
-  const int l = threadIdx.x & 63;
+  }
+  // Row l is tile l / 32's: the halves exchange what the other's rows need, then each lane adds its row's shares
+  // in the order of the units.
   float y = 0.0f;
-  for (int h = 0; h < kHid; ++h) y += from_bf16(to_bf16(silu(s.z2[l * kS32 + h]))) * w.w3[h];
-  return y + w.b3;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    float lo[4], hi[4];  // units 8 q + 0 .. 3 and 8 q + 4 .. 7
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const auto both = __builtin_amdgcn_permlane32_swap(part[0][4 * q + i], part[1][4 * q + i], false, false);
+      const uint32_t a = both[0], b = both[1];
+      lo[i] = __builtin_bit_cast(float, a);
+      hi[i] = __builtin_bit_cast(float, b);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y += lo[i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y += hi[i];
+  }
+  wave_sync();  // (the next call's features overwrite xs)
+  return y + s.b3;
 }
 
 }  // namespace mlp

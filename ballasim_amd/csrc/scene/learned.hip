@@ -262,15 +262,18 @@ __global__ __launch_bounds__(256) void learned_init_kernel(SceneDev sc, ViewDev 
 
 // One window (t_w, t_w + W] of every pixel. kWrite false: counts[p] = the pixel's samples and the
 // work counters; true: the samples at row_start[p] and the new controller state.
+// Bound by the latency of each lane's chain of decisions (features, network, two renders, check), so by the waves
+// in flight: the network's activations in registers (15 KB of LDS a wave, where 64 KB let two waves share a compute
+// unit) and the weights loaded only where a shape passes took a 1280x720 window with 12 disks from 2.03 ms a pass to
+// 1.05-1.15; registers held to two waves per SIMD (256 with the accumulators, where 220 and the accumulators let one
+// run) to 0.81 (write) and 1.0 (count).
 template <bool kWrite>
-__global__ __launch_bounds__(64) void learned_window_kernel(SceneDev sc, ViewDev view, LearnedRules r, const uint16_t* wb,
-                                                            const float* w, int64_t t_w, LearnedState st,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void learned_window_kernel(
+    SceneDev sc, ViewDev view, LearnedRules r, const uint16_t* wb, const float* w, int64_t t_w, LearnedState st,
                                                             SensorLink link, int32_t* counts,
                                                             const int64_t* row_start, int64_t* t_out, float* irr_out,
                                                             unsigned long long* work) {
-  __shared__ mlp::WeightsLds W;
-  __shared__ mlp::WaveLds S;
-  mlp::load_weights(W, wb, w);
+  __shared__ mlp::WaveWeights W;
   const uint32_t P = view.width * view.height;
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = p < P;
@@ -330,13 +333,13 @@ __global__ __launch_bounds__(64) void learned_window_kernel(SceneDev sc, ViewDev
     h.push(ts, e, sg, log_irr(e, r.dark), r.dark);
   };
   const auto at = [&](int64_t ts) { return eval_scene(sc, mask, x, y, static_cast<double>(ts) * 1e-9); };
+  if (__ballot(active) != 0) mlp::load_weights(W, wb, w);  // (a block is one wave; most see no shape)
   while (__ballot(active) != 0) {
     float f[kIn];
     if (active) features(h, r.theta_band, f);
     else
       for (int c = 0; c < kIn; ++c) f[c] = 0.0f;
-    mlp::put_features(S, f);
-    const float out = mlp::wave_forward(W, S);
+    const float out = mlp::wave_forward(W, f);
     if (active) {
       ++proposals;
       const double dt_pred = exp(2.0 * static_cast<double>(out) + kLnDtCenter) * r.margin;

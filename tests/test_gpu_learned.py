@@ -116,6 +116,46 @@ def test_learned_controller_gain():
     assert out["learned"]["count_mismatch"] < 0.01
 
 
+# A pixel's samples depend on its own light alone: views of one pixel, a row of one fewer and one more than a
+# wave, and a ragged block, laid around the pixel of the most samples, give the samples of the same pixels of the
+# whole view, to the bit, wherever their lanes are and whichever lanes of their wave are at work.
+@pytest.mark.parametrize("w,h", [(1, 1), (63, 1), (65, 1), (37, 41)])
+def test_samples_do_not_depend_on_the_lane(w, h):
+    import ballasim_amd as bsx
+    from ballasim_amd import scene as S
+    from ballasim_amd.learned import LearnedSampler, Proposer, learned_rules
+    p = _sensor_params(bsx)
+    dark = float(p.dark_current_fA) / float(p.illuminance_scale)
+    sc, v = S.learned_eval_scene(3, 640, 360, 8)
+    prop = Proposer(5)
+    rules = learned_rules(S.rules(dark, tol=0.01), tol_log=0.01, theta_band=0.2, margin=0.5, near=0.05)
+
+    def rows(view):
+        ls = LearnedSampler(sc, view, rules, prop)
+        ls.init(0)
+        out = []
+        for i in range(3):
+            ids, ts, ir, offs = S.runs_to_host(ls.window(i * W, slot=0)[0])
+            out.append({int(px): (ts[a:b], ir[a:b]) for px, a, b in zip(ids, offs[:-1], offs[1:]) if b > a})
+        return out
+
+    whole = rows(v)
+    most = max(whole[0], key=lambda px: len(whole[0][px][0]))
+    x0 = min(max(most % v.width - w // 3, 0), v.width - w)
+    y0 = min(max(most // v.width - h // 3, 0), v.height - h)
+    part = rows(S.view(w, h, v.origin_x + x0 * v.px_scale, v.origin_y + y0 * v.px_scale, v.px_scale))
+    for big, small in zip(whole, part):
+        want = {}
+        for px, row in big.items():
+            x, y = px % v.width - x0, px // v.width - y0
+            if 0 <= x < w and 0 <= y < h:
+                want[y * w + x] = row
+        assert want.keys() == small.keys()
+        for px, (ts, ir) in want.items():
+            assert np.array_equal(ts, small[px][0]) and np.array_equal(ir, small[px][1]), px
+    assert len(part[0]) > 0
+
+
 def test_learned_gain_at_equal_error_config4():
     """Config 4 at its own workload: the proposer trained on 20 M dense-trace examples of 20 seeded
     scenes, then the learned controller against the plain one at 1280x720 over 503 ms (60 windows)
