@@ -535,9 +535,11 @@ CameraDev SensorModel::stage(const RunsDev& runs, const uint32_t* pixel, size_t 
   bool coefs = false;
   if (!inst && !noise_ && total > 0) {
     // the cascade's segment coefficients: 24 bytes per segment, left out (the walk then forms them itself)
-    // past kMaxCoefBytes or when the device has no room for them
+    // past kMaxCoefBytes or a quarter of the free device memory, which is the caller's to use
     const size_t bytes = static_cast<size_t>(total) * sizeof(SegmentCoef);
-    if (bytes <= kMaxCoefBytes) {
+    size_t free_bytes = 0, all_bytes = 0;
+    if (bytes <= d_coefs_.bytes() ||
+        (bytes <= kMaxCoefBytes && hipMemGetInfo(&free_bytes, &all_bytes) == hipSuccess && bytes <= free_bytes / 4)) {
       try {
         d_coefs_.ensure(bytes);
         coefs = true;
