@@ -188,3 +188,41 @@ def test_output_order_of_any_size(n, size, readout, span):
                      ("t_reported_ns", "t_reported"), ("t_cross_ns", "t_cross"), ("label", "label"), ("flags", "flags")):
             assert np.array_equal(got[a], want[b]), a
     assert stage.held == 0
+
+
+# A column copy by several threads (more than two 1 MiB chunks) behind the columns' kernel, whatever stream the caller
+# names: the null stream, one of its own, and the handle that names another stream in each thread. The second window
+# differs from the first, whose columns the stage's buffers still hold.
+@pytest.mark.parametrize("kind", ["null", "own", "per_thread"])
+def test_columns_on_any_stream(kind):
+    import torch
+
+    import ballasim_amd as bsx
+    from ballasim_amd.output import OutputStage
+    p = bsx.preset("prophesee_gen3")
+    p.photoreceptor = "instantaneous"
+    p.noise = False
+    Wd, Hd, n = 640, 480, 200000
+    m = bsx.SensorModel(p, Wd, Hd, 3, ["constant"], 0, device="cuda")
+    rd = dict(quantum=round(p.readout_quantum_s * 1e9), delay=round(p.readout_delay_s * 1e9),
+              phase=int(m._info().readout_phase_ns), offset=int(p.clock_offset_ns), drift_ppm=float(p.clock_drift_ppm))
+    own = torch.cuda.Stream()
+    stream = {"null": 0, "own": own, "per_thread": 2}[kind]  # 2: hipStreamPerThread
+    stage, oracle = OutputStage(m), Q.OutputOracle(Wd, Hd, rd)
+    rng = np.random.default_rng(3)
+    for w in range(2):
+        ev = np.zeros(n, RAW_EVENT)
+        ev["pixel"] = rng.integers(0, Wd * Hd, n)
+        ev["polarity"] = rng.integers(0, 2, n)
+        ev["label"] = rng.integers(0, 4, n)
+        ev["t_cross"] = w * W + 1 + rng.permutation(n) * (W // n)
+        raw = np.zeros(n, O.EVENT_DTYPE)
+        for f in ("pixel", "polarity", "label", "flags", "t_cross"):
+            raw[f] = ev[f]
+        dev = torch.from_numpy(ev.view(np.uint8).reshape(n, 32)).cuda()
+        torch.cuda.synchronize()
+        got, want = stage.window((dev.data_ptr(), n), w * W, stream=stream), oracle.window(raw, w * W)
+        assert len(got["t"]) == len(want["t"]) > 100000
+        for a, b in (("x", "x"), ("y", "y"), ("p", "p"), ("t", "t"), ("t_ns_rem", "t_ns_rem"),
+                     ("t_reported_ns", "t_reported"), ("t_cross_ns", "t_cross"), ("label", "label"), ("flags", "flags")):
+            assert np.array_equal(got[a], want[b]), (w, a)
