@@ -4,11 +4,10 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <mutex>
 #include <stdexcept>
 #include <string>
-#include <thread>
 
+#include "../core/workers.h"
 #include "output_kernels.h"
 
 namespace bsx {
@@ -264,20 +263,11 @@ void OutputStage::copy_out(const char* from, const std::vector<Piece>& dst, size
   hip_check(hipGetDevice(&device), "device");
   const size_t n_threads = std::min<size_t>(kCopyThreads, (chunks + 1) / 2);
   std::atomic<int> error{hipSuccess};
-  const auto work = [&](size_t k) {
+  run_workers(n_threads, [&](size_t k) noexcept {
     hipError_t e = hipSetDevice(device);
     if (e == hipSuccess) e = run(k, n_threads, staging_ + 2 * k * kCopyBytes, copy_);
     if (e != hipSuccess) error.store(e);
-  };
-  std::vector<std::thread> pool;
-  size_t started = 1;
-  try {
-    for (; started < n_threads; ++started) pool.emplace_back(work, started);
-  } catch (const std::system_error&) {  // no more threads: this one takes their chunks
-  }
-  for (size_t k = started; k < n_threads; ++k) work(k);
-  work(0);
-  for (std::thread& t : pool) t.join();
+  });
   hip_check(static_cast<hipError_t>(error.load()), "download columns");
 }
 
