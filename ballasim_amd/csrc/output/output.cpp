@@ -280,6 +280,7 @@ void OutputStage::fetch(const OutputColumnsDst& d, hipStream_t stream) {
   char* const first = b;
   std::vector<Piece> pieces;
   const auto column = [&](auto* to) {
+    if (to == nullptr) throw std::invalid_argument("OutputStage.fetch: null column");
     using T = std::remove_pointer_t<decltype(to)>;
     T* at = reinterpret_cast<T*>(b);
     b += m * sizeof(T);

@@ -55,7 +55,9 @@ int bsx_output_window(bsx_output* o, const bsx_device_events* events, int64_t t_
 int bsx_output_flush(bsx_output* o, void* stream, bsx_output_events* out);
 
 /* The same two calls with the released events left on the device, and their columns fetched into the caller's own
- * host arrays (each with room for *released events) before the stage's next call. */
+ * host arrays (each with room for *released events, none null) before the stage's next call. A stage whose columns
+ * once exceeded 2 MiB (61,680 events) holds 12 MiB of pinned host memory for their copies until it is destroyed, others
+ * that fetched 2 MiB. */
 typedef struct bsx_output_columns {
   uint16_t* x;
   uint16_t* y;

@@ -226,3 +226,37 @@ def test_columns_on_any_stream(kind):
         for a, b in (("x", "x"), ("y", "y"), ("p", "p"), ("t", "t"), ("t_ns_rem", "t_ns_rem"),
                      ("t_reported_ns", "t_reported"), ("t_cross_ns", "t_cross"), ("label", "label"), ("flags", "flags")):
             assert np.array_equal(got[a], want[b]), (w, a)
+
+
+@pytest.mark.parametrize("missing", ["x", "t", "flags"])
+def test_fetch_refuses_a_null_column(missing):
+    import ctypes as C
+
+    import torch
+
+    import ballasim_amd as bsx
+    from ballasim_amd import _abi
+    from ballasim_amd.output import _COLUMNS, OutputColumns, OutputStage
+    p = bsx.preset("prophesee_gen3")
+    p.photoreceptor = "instantaneous"
+    p.noise = False
+    m = bsx.SensorModel(p, 40, 24, 3, ["constant"], 0, device="cuda")
+    stage = OutputStage(m)
+    ev = np.zeros(100, RAW_EVENT)
+    ev["pixel"] = np.arange(100)
+    ev["t_cross"] = 1 + 10000 * np.arange(100)  # (each with a report of its own)
+    dev = torch.from_numpy(ev.view(np.uint8).reshape(100, 32)).cuda()
+    torch.cuda.synchronize()
+    n, held = C.c_size_t(), C.c_size_t()
+    lib = _abi.load_library()
+    _abi.check(lib.bsx_output_window_count(stage._h, C.byref(_abi.DeviceEvents(dev.data_ptr(), 100)), 0, None,
+                                           C.byref(n), C.byref(held)))
+    assert n.value == 100
+    cols = {name: np.zeros(100, dt) for name, dt in _COLUMNS}
+    ptr = [None if name == missing else a.ctypes.data for name, a in cols.items()]
+    with pytest.raises(ValueError, match="null column"):
+        _abi.check(lib.bsx_output_fetch(stage._h, None, C.byref(OutputColumns(*ptr))))
+    # refused before anything is written, and the events are still there to fetch
+    assert all(not a.any() for a in cols.values())
+    _abi.check(lib.bsx_output_fetch(stage._h, None, C.byref(OutputColumns(*[a.ctypes.data for a in cols.values()]))))
+    assert np.array_equal(cols["x"], np.arange(100) % 40) and np.array_equal(cols["t_cross_ns"], ev["t_cross"])
