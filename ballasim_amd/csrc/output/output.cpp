@@ -12,19 +12,6 @@
 
 namespace bsx {
 
-namespace {
-
-int bit_length(uint64_t v) {
-  int b = 0;
-  while (v != 0) {
-    ++b;
-    v >>= 1;
-  }
-  return b;
-}
-
-}  // namespace
-
 void OutputColumns::resize(size_t n) {
   x.resize(n);
   y.resize(n);
@@ -127,11 +114,12 @@ size_t OutputStage::release_sorted(size_t total, int64_t cut, hipStream_t stream
   const int64_t lag_min = unbias(kOutLagMin), lag_max = unbias(kOutLagMax);
   const OutEventDev* ev = held_.as<const OutEventDev>();
   sorted_.ensure(total * sizeof(OutEventDev));
-  OrderKey key{tr_min, lag_min, bit_length(static_cast<uint64_t>(tr_max) - static_cast<uint64_t>(tr_min)), x_bits_,
-               y_bits_, bit_length(static_cast<uint64_t>(lag_max) - static_cast<uint64_t>(lag_min))};
+  const OrderKey key = order_key_of(readout_, tr_min, tr_max, lag_min, lag_max, x_bits_, y_bits_);
   bool done = false;
   if (key.bits() <= 64) {
-    const int bb = out_bucket_bits(total);
+    const int bb = out_bucket_bits(total, key, report_count(readout_, tr_min, tr_max),
+                                   crop_on_ ? static_cast<uint32_t>(crop_.x1 - crop_.x0) : width_,
+                                   crop_on_ ? static_cast<uint32_t>(crop_.y1 - crop_.y0) : height_);
     if (bb > 0) {
       keys_.ensure(total * 8);
       perm_.ensure(total * 4);
@@ -142,7 +130,7 @@ size_t OutputStage::release_sorted(size_t total, int64_t cut, hipStream_t stream
                                  stream),
               "bucket sort");
     read_scratch(stream);
-    done = bb == 0 || h_scratch_[kOutMostBucket] <= out_bucket_cap();
+    done = bb == 0 || h_scratch_[kOutMostBucket] <= kBucketCap;
   }
   if (!done) {
     sort_digits(total, cut, tr_min, tr_max, tr_min + lag_min, tr_max + lag_max, stream);

@@ -129,23 +129,14 @@ __global__ __launch_bounds__(kOutBlock) void build_kernel(const RawEventDev* raw
 
 // ---- The bucket sort -----------------------------------------------------------------------------
 // The output order is the order of one integer key (OrderKey: t_reported, x, y and the lag t_cross -
-// t_reported, each less its minimum), unique per event. Its leading bits part the events into buckets of a few
+// t_reported), unique per event. Its leading bits part the events into buckets of a few
 // hundred (reported times spread over the window), counted and filled with one atomic per event, and one block
 // per bucket sorts its keys in LDS and writes the events in order: four short passes whatever the key's
 // length, where the digit sort below makes ten of five kernels each (2.9 M events: 0.58 ms of kernels, and
 // 50 launches in a window of any size). Keys of more than 64 bits, and a bucket of more than kBucketCap events
-// (coarse readouts), are left to the digit sort.
-constexpr int kBucketCap = 2048;
-
+// (bursts), are left to the digit sort.
 __device__ __forceinline__ uint64_t order_key(const OrderKey& k, const OutEventDev& o) {
-  return (((((static_cast<uint64_t>(o.t_reported - k.rep_min) << k.x_bits) | o.x) << k.y_bits) | o.y) << k.lag_bits) |
-         static_cast<uint64_t>((o.t_cross - o.t_reported) - k.lag_min);
-}
-
-// (clamped: an event outside the frame has a key past the others')
-__device__ __forceinline__ uint32_t bucket_of(uint64_t key, int shift, uint32_t buckets) {
-  const uint64_t b = key >> shift;
-  return b < buckets ? static_cast<uint32_t>(b) : buckets - 1;
+  return order_key(k, o.t_reported, o.x, o.y, o.t_cross);
 }
 
 __global__ __launch_bounds__(256) void bucket_count_kernel(const OutEventDev* ev, size_t n, OrderKey k, int shift,
@@ -400,14 +391,6 @@ hipError_t launch_out_build(const RawEventDev* raw, size_t n, uint32_t width, co
   }
   return hipGetLastError();
 }
-
-int out_bucket_bits(size_t n) {
-  int b = 0;
-  while (n > kBucketCap && (n >> b) > 512 && b < kMaxBucketBits) ++b;
-  return b;
-}
-
-size_t out_bucket_cap() { return kBucketCap; }
 
 hipError_t launch_out_buckets(const OutEventDev* ev, size_t n, const OrderKey& k, int bucket_bits, int64_t cut,
                               uint32_t* words, uint64_t* keys, uint32_t* perm, OutEventDev* sorted,

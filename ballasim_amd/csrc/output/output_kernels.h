@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "order_key.h"
 #include "output.h"
 
 namespace bsx {
@@ -11,24 +12,13 @@ namespace bsx {
 // held and new events (biased to unsigned order), the released events, the largest bucket.
 enum OutScratch : int { kOutKept, kOutRepMin, kOutRepMax, kOutLagMin, kOutLagMax, kOutReady, kOutMostBucket, kOutScratch };
 
-// The integer whose order is the output order: t_reported - rep_min, x, y and the lag t_cross - t_reported less
-// lag_min, from the leading bits down.
-struct OrderKey {
-  int64_t rep_min, lag_min;
-  int32_t rep_bits, x_bits, y_bits, lag_bits;
-  BSX_HD int bits() const { return rep_bits + x_bits + y_bits + lag_bits; }
-};
-inline constexpr int kMaxBucketBits = 14;
-
 // Resets scratch, appends the kept raw events as OutEventDev at held[n_held ..] and folds the extremes.
 hipError_t launch_out_build(const RawEventDev* raw, size_t n, uint32_t width, const Readout& r, bool crop,
                             const CropBox& box, OutEventDev* held, size_t n_held, unsigned long long* scratch,
                             hipStream_t stream);
 // The bucket sort of ev[0 .. n) into sorted by a key of at most 64 bits, the events reported before cut counted:
-// 2^bucket_bits buckets (out_bucket_bits(n); 0: n events fit one block), words holds 3 << bucket_bits. Complete
-// when the largest bucket (scratch) is at most out_bucket_cap().
-int out_bucket_bits(size_t n);
-size_t out_bucket_cap();
+// 2^bucket_bits buckets (out_bucket_bits; 0: n events fit one block), words holds 3 << bucket_bits. Complete
+// when the largest bucket (scratch) is at most kBucketCap.
 hipError_t launch_out_buckets(const OutEventDev* ev, size_t n, const OrderKey& k, int bucket_bits, int64_t cut,
                               uint32_t* words, uint64_t* keys, uint32_t* perm, OutEventDev* sorted,
                               unsigned long long* scratch, hipStream_t stream);

@@ -142,15 +142,18 @@ RAW_EVENT = np.dtype([("pixel", np.uint32), ("polarity", np.uint8), ("label", np
                       ("l_first", np.float32)])
 
 
-# One block's sort and its edges, the first sizes that are bucketed, a quantum so coarse that buckets overflow
-# (the digit sort takes over), a drift that gives neighbouring times one report, keys of more than 64 bits, and a
-# column copy of several chunks.
+# One block's sort and its edges, the first sizes that are bucketed, quanta that the key divides out (up to two reports
+# a window), a drift that gives neighbouring times one report, keys of more than 64 bits (the digit sort), and a column
+# copy of several chunks.
 @pytest.mark.parametrize("n,size,readout,span", [
     (1, (3, 2), {}, W), (2, (3, 2), {}, 3), (63, (40, 24), {}, W), (65, (40, 24), dict(readout_quantum_s=1e-6), W),
     (2048, (640, 480), dict(readout_quantum_s=2e-5), W), (2049, (640, 480), {}, W),
     (30000, (2048, 1536), dict(readout_quantum_s=5e-3), W), (30000, (64, 48), dict(readout_quantum_s=0.0,
      clock_drift_ppm=-4000.0), 60000), (5000, (65535, 3), dict(readout_quantum_s=1.0), 1 << 40),
-    (300001, (1280, 720), dict(readout_quantum_s=1e-6, clock_drift_ppm=35.0), W)])
+    (300001, (1280, 720), dict(readout_quantum_s=1e-6, clock_drift_ppm=35.0), W),
+    (5000, (65535, 3), dict(readout_quantum_s=0.0, clock_drift_ppm=-4000.0), 1 << 40),
+    (200000, (1280, 720), dict(readout_quantum_s=2e-5), W),
+    (200000, (1280, 720), dict(readout_quantum_s=1e-3, clock_drift_ppm=35.0), W)])
 def test_output_order_of_any_size(n, size, readout, span):
     import torch
 
