@@ -38,7 +38,7 @@ inline int bit_length(uint64_t v) {
 // product off by at most 2^12 |drift| ns for any 64-bit time), so those whose quotients by 2^shift <= gap are equal
 // are equal. With the raw nanoseconds as the key's leading bits a quantum of 20 us put a window's 2.9 M events into
 // 1 of 40 buckets, each past what a block sorts, and the digit sort ran after all (a window and its flush to a stream
-// 2.26 ms, 0.98 this way, 1.52 by the digit sort alone; at 1 ms 1.46, 1.27 and 1.50).
+// 2.26 ms, 0.98 this way, 1.52 by the digit sort alone; at 1 ms 1.46, 1.27 and 1.51).
 inline int report_shift(const Readout& r) {
   if (r.quantum_ns <= 1) return 0;
   const double drift = r.clock_drift_ppm * 1e-6;
@@ -74,22 +74,22 @@ inline double report_count(const Readout& r, int64_t rep_min, int64_t rep_max) {
 // The buckets of n events (as a power of two; 0: one block takes them all): as many as leave 512 to each bucket that
 // events of `reports` reported times and a crop of width x height pixels can reach. (Of a field that the bucket's bits
 // touch only the values in use are reached: of 2,048 buckets that 900,000 events over 1280x720 and nine reports were
-// parted into, 360.)
+// parted into, 360.) -1: more events than blocks could sort if they were spread evenly, the digit sort's (20 M events
+// over 8 ms and 2048x1536 pixels took 10.4 ms with the bucket passes in vain, 7.2 without).
 inline int out_bucket_bits(size_t n, const OrderKey& k, double reports, uint32_t width, uint32_t height) {
   if (n <= kBucketCap) return 0;
   const auto share = [](double values, int bits) {
     return bits >= 63 ? 1.0 : vmin(1.0, values / static_cast<double>(int64_t{1} << bits));
   };
-  int b = 0;
-  while (b < kMaxBucketBits) {
+  for (int b = 1; b <= kMaxBucketBits; ++b) {
     double reached = static_cast<double>(1 << b);
-    if (b > 0) reached *= share(reports, k.rep_bits);
+    reached *= share(reports, k.rep_bits);
     if (b > k.rep_bits) reached *= share(width, k.x_bits);
     if (b > k.rep_bits + k.x_bits) reached *= share(height, k.y_bits);
-    if (b > 0 && static_cast<double>(n) <= 512.0 * reached) break;
-    ++b;
+    if (static_cast<double>(n) <= 512.0 * reached) return b;
+    if (b == kMaxBucketBits && static_cast<double>(n) > static_cast<double>(kBucketCap) * reached) return -1;
   }
-  return b;
+  return kMaxBucketBits;
 }
 
 // (clamped: an event outside the frame has a key past the others')

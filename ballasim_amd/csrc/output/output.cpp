@@ -115,11 +115,12 @@ size_t OutputStage::release_sorted(size_t total, int64_t cut, hipStream_t stream
   const OutEventDev* ev = held_.as<const OutEventDev>();
   sorted_.ensure(total * sizeof(OutEventDev));
   const OrderKey key = order_key_of(readout_, tr_min, tr_max, lag_min, lag_max, x_bits_, y_bits_);
+  const int bb = key.bits() > 64 ? -1
+                                 : out_bucket_bits(total, key, report_count(readout_, tr_min, tr_max),
+                                                   crop_on_ ? static_cast<uint32_t>(crop_.x1 - crop_.x0) : width_,
+                                                   crop_on_ ? static_cast<uint32_t>(crop_.y1 - crop_.y0) : height_);
   bool done = false;
-  if (key.bits() <= 64) {
-    const int bb = out_bucket_bits(total, key, report_count(readout_, tr_min, tr_max),
-                                   crop_on_ ? static_cast<uint32_t>(crop_.x1 - crop_.x0) : width_,
-                                   crop_on_ ? static_cast<uint32_t>(crop_.y1 - crop_.y0) : height_);
+  if (bb >= 0) {
     if (bb > 0) {
       keys_.ensure(total * 8);
       perm_.ensure(total * 4);
@@ -130,7 +131,7 @@ size_t OutputStage::release_sorted(size_t total, int64_t cut, hipStream_t stream
                                  stream),
               "bucket sort");
     read_scratch(stream);
-    done = bb == 0 || h_scratch_[kOutMostBucket] <= kBucketCap;
+    done = h_scratch_[kOutMostBucket] <= kBucketCap;
   }
   if (!done) {
     sort_digits(total, cut, tr_min, tr_max, tr_min + lag_min, tr_max + lag_max, stream);

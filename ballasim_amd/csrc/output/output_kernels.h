@@ -17,7 +17,7 @@ hipError_t launch_out_build(const RawEventDev* raw, size_t n, uint32_t width, co
                             const CropBox& box, OutEventDev* held, size_t n_held, unsigned long long* scratch,
                             hipStream_t stream);
 // The bucket sort of ev[0 .. n) into sorted by a key of at most 64 bits, the events reported before cut counted:
-// 2^bucket_bits buckets (out_bucket_bits; 0: n events fit one block), words holds 3 << bucket_bits. Complete
+// 2^bucket_bits buckets (0: n events fit one block), words holds 3 << bucket_bits. Complete
 // when the largest bucket (scratch) is at most kBucketCap.
 hipError_t launch_out_buckets(const OutEventDev* ev, size_t n, const OrderKey& k, int bucket_bits, int64_t cut,
                               uint32_t* words, uint64_t* keys, uint32_t* perm, OutEventDev* sorted,

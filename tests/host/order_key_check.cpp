@@ -105,6 +105,10 @@ static int fill(size_t n, uint32_t w, uint32_t h, int64_t quantum, double drift)
   int64_t r0 = INT64_MAX, r1 = INT64_MIN;
   for (const Event& e : ev) r0 = std::min(r0, e.rep), r1 = std::max(r1, e.rep);
   const int bb = bsx::out_bucket_bits(n, q, bsx::report_count(r, r0, r1), w, h);
+  if (bb < 0) {
+    std::printf("too many\n");
+    return 0;
+  }
   const int shift = std::max(0, q.bits() - bb);
   std::vector<uint32_t> count(size_t{1} << bb);
   for (const Event& e : ev) ++count[bsx::bucket_of(bsx::order_key(q, e.rep, e.x, e.y, e.cross), shift, 1u << bb)];

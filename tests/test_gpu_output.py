@@ -263,3 +263,37 @@ def test_fetch_refuses_a_null_column(missing):
     assert all(not a.any() for a in cols.values())
     _abi.check(lib.bsx_output_fetch(stage._h, None, C.byref(OutputColumns(*[a.ctypes.data for a in cols.values()]))))
     assert np.array_equal(cols["x"], np.arange(100) % 40) and np.array_equal(cols["t_cross_ns"], ev["t_cross"])
+
+
+# Bursts: buckets past what a block sorts leave the events to the digit sort, with a window's other events around them
+# or not; the largest that still fits, and one event more.
+@pytest.mark.parametrize("burst,spread", [(2048, 700), (2049, 700), (60000, 700), (60000, 0), (300000, 50000)])
+def test_bursts(burst, spread):
+    import torch
+
+    import ballasim_amd as bsx
+    from ballasim_amd.output import OutputStage
+    p = bsx.preset("prophesee_gen3")
+    p.photoreceptor = "instantaneous"
+    p.noise = False
+    p.readout_quantum_s = 0.0
+    Wd, Hd = 1280, 720
+    m = bsx.SensorModel(p, Wd, Hd, 3, ["constant"], 0, device="cuda")
+    rd = dict(quantum=0, delay=round(p.readout_delay_s * 1e9), phase=0, offset=int(p.clock_offset_ns),
+              drift_ppm=float(p.clock_drift_ppm))
+    rng = np.random.default_rng(burst)
+    n = burst + spread
+    ev = np.zeros(n, RAW_EVENT)
+    ev["pixel"] = rng.permutation(Wd * Hd)[:n]
+    ev["polarity"] = rng.integers(0, 2, n)
+    ev["t_cross"] = np.where(rng.permutation(n) < burst, 3000000 + rng.integers(0, 2, n), 1 + rng.integers(0, W - 1, n))
+    stage, oracle = OutputStage(m), Q.OutputOracle(Wd, Hd, rd)
+    dev = torch.from_numpy(ev.view(np.uint8).reshape(n, 32)).cuda()
+    torch.cuda.synchronize()
+    raw = np.zeros(n, O.EVENT_DTYPE)
+    for f in ("pixel", "polarity", "label", "flags", "t_cross"):
+        raw[f] = ev[f]
+    for got, want in ((stage.window((dev.data_ptr(), n), 0), oracle.window(raw, 0)), (stage.flush(), oracle.flush())):
+        for a, b in (("x", "x"), ("y", "y"), ("p", "p"), ("t_reported_ns", "t_reported"), ("t_cross_ns", "t_cross")):
+            assert np.array_equal(got[a], want[b]), a
+    assert stage.held == 0

@@ -40,3 +40,12 @@ def test_buckets_fit_a_block_at_any_quantum(order_key_check, n, size, drift, qua
                        capture_output=True, text=True, timeout=120)
     largest, cap = map(int, re.search(r"largest (\d+) cap (\d+)", r.stdout).groups())
     assert largest <= cap, r.stdout
+
+
+# Where even events spread evenly are too many for blocks to sort, the bucket passes are not tried; below, they are.
+@pytest.mark.parametrize("n,size,quantum_ns,tried", [(2049, (3, 2), 0, True), (8000000, (2048, 1536), 1000, True),
+                                                     (20000000, (2048, 1536), 1000, False)])
+def test_bucket_passes_are_not_tried_in_vain(order_key_check, n, size, quantum_ns, tried):
+    r = subprocess.run([str(order_key_check), "fill", str(n), str(size[0]), str(size[1]), str(quantum_ns), "0"],
+                       capture_output=True, text=True, timeout=120)
+    assert ("too many" not in r.stdout) == tried, r.stdout
