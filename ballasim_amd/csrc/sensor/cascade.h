@@ -412,8 +412,11 @@ BSX_HD BSX_INLINE TryCoef try_coef(const Consts& cc, float I_a, float I_b, float
   return q;
 }
 
-// The range of the comparator input over an accepted sub-step up to roundings (the cubic's hull and the
-// free modes' end values).
+// The range of s3 over an accepted sub-step (the cubic's hull and the free modes' end values), widened by kHullSlack
+// times the sum of its terms' magnitudes: more than the roundings of this range and of the values the exact test and
+// its search form of the same terms (some twenty roundings of 2^-24 on the largest, three times that where the cubic
+// is shifted). With far apart time constants the terms of the non-residual form cancel from 1e5 and more.
+constexpr float kHullSlack = 0x1p-17f;
 struct Hull {
   float lo, hi;
 };
@@ -491,8 +494,10 @@ BSX_HD BSX_INLINE bool try_substep(const Consts& cc, const State& st, float i_sc
     const float e1 = g.c[1] * h, e2 = g.c[2] * h * h, e3 = g.c[3] * h * h * h;
     const float b1 = e1 * (1.0f / 3.0f), b2 = (2.0f * e1 + e2) * (1.0f / 3.0f), b3 = e1 + e2 + e3;
     const float s0 = resid ? 0.0f : g.C[0], s1 = resid ? 0.0f : g.C[1], f0 = g.C[0] * r2, f1 = g.C[1] * r3;
-    hull.lo = g.c[0] + vmin(vmin(0.0f, b1), vmin(b2, b3)) + vmin(s0, f0) + vmin(s1, f1);
-    hull.hi = g.c[0] + vmax(vmax(0.0f, b1), vmax(b2, b3)) + vmax(s0, f0) + vmax(s1, f1);
+    const float slack = kHullSlack * (fabs_(g.c[0]) + fabs_(e1) + fabs_(e2) + fabs_(e3) + vmax(fabs_(s0), fabs_(f0)) +
+                                      vmax(fabs_(s1), fabs_(f1)));
+    hull.lo = g.c[0] + vmin(vmin(0.0f, b1), vmin(b2, b3)) + vmin(s0, f0) + vmin(s1, f1) - slack;
+    hull.hi = g.c[0] + vmax(vmax(0.0f, b1), vmax(b2, b3)) + vmax(s0, f0) + vmax(s1, f1) + slack;
   }
   sub.x1_a = x1a;
   sub.x1_b = x1b;
@@ -561,16 +566,17 @@ struct CascadeLane : InstantLane<kMaxG, 2> {
 
   BSX_HD BSX_INLINE float s3_in(int64_t t) const { return s3_fn_(static_cast<float>(t - (pc_.t_a + cmp_a_)) * 1e-9f); }
 
-  // True when the sub-step is finished. The hull, formed with a few more roundings than the exact test
-  // (each below 1e-6 of the terms, which stay below the levels plus 128), bounds the comparator input on
-  // the whole sub-step, so with a margin of 2^-10 no integer of it fires: the exact test or the search
-  // behind it says the same, and leaves the same state.
+  // True when the sub-step is finished: the hull of s3, moved by the reference and the leak with a margin of
+  // 2^-10 and of kHullSlack times what moves it, lies inside the levels, so no integer of the sub-step fires;
+  // the exact test or the search behind it says the same, and leaves the same state.
   BSX_HD BSX_INLINE bool compare_quick() {
     const int64_t t_a = pc_.t_a + cmp_a_, t_b = pc_.t_a + cmp_b_;
     if (blind_until != kNotBlind) return blind_until >= t_b;
     if (t_search >= t_b) return true;
-    const float base = leak * ns_to_s64<float>(t_a - t_ref) + dr_ref - s3_ref;
-    const float rise = fabs_(leak) * (static_cast<float>(cmp_b_ - cmp_a_) * 1e-9f) + 0x1p-10f;
+    const float drift = leak * ns_to_s64<float>(t_a - t_ref);
+    const float base = drift + dr_ref - s3_ref;
+    const float rise = fabs_(leak) * (static_cast<float>(cmp_b_ - cmp_a_) * 1e-9f) + 0x1p-10f +
+                       cascade::kHullSlack * (fabs_(drift) + fabs_(dr_ref) + fabs_(s3_ref));
     if (!(hull_.hi + base + rise < theta_on && hull_.lo + base - rise > -theta_off)) return false;
     ++n_leaves;
     t_search = t_b;
