@@ -8,6 +8,7 @@
 #include <string>
 
 #include "chain.h"
+#include "coefs.h"
 #include "kernels.h"
 #include "noise_tables.h"
 #include "scratch.h"
@@ -19,7 +20,6 @@ namespace {
 constexpr double kMaxSamplePhotocurrent_fA = 1e9;  // the reference's input clamp (src/sensor/pixel.h:97)
 constexpr uint32_t kStateMagic = 0x534e5342;      // "BSNS"
 constexpr uint32_t kStateVersion = 6;
-constexpr size_t kMaxCoefBytes = size_t{32} << 30;  // of segment coefficients per camera
 
 struct StateHeader {
   uint32_t magic, version;
@@ -532,14 +532,16 @@ CameraDev SensorModel::stage(const RunsDev& runs, const uint32_t* pixel, size_t 
   d_events_.ensure(cap_ * sizeof(RawEventDev));
   d_work_.ensure(std::max<size_t>(n_runs, 1) * sizeof(float));
   d_loud_.ensure(std::max<size_t>(n_runs, 1) * sizeof(int));
-  bool coefs = false;
+  bool coefs = false;  // the cascade's segment coefficients: 24 bytes per segment, or none
   if (!inst && !noise_ && total > 0) {
-    // the cascade's segment coefficients: 24 bytes per segment, left out (the walk then forms them itself)
-    // past kMaxCoefBytes or a quarter of the free device memory, which is the caller's to use
-    const size_t bytes = static_cast<size_t>(total) * sizeof(SegmentCoef);
+    const size_t need = static_cast<size_t>(total) * sizeof(SegmentCoef), have = d_coefs_.bytes();
     size_t free_bytes = 0, all_bytes = 0;
-    if (bytes <= d_coefs_.bytes() ||
-        (bytes <= kMaxCoefBytes && hipMemGetInfo(&free_bytes, &all_bytes) == hipSuccess && bytes <= free_bytes / 4)) {
+    if (need > have && hipMemGetInfo(&free_bytes, &all_bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      free_bytes = 0;
+    }
+    const size_t bytes = coef_bytes(need, have, free_bytes);
+    if (bytes > 0) {
       try {
         d_coefs_.ensure(bytes);
         coefs = true;
