@@ -1227,9 +1227,8 @@ __device__ __forceinline__ void cascade_lanes(const CameraDev* cams, int n_cams,
 // with the coefficients 3.9, against 29.5 and 1.2 with one pixel per lane, each lane forming its own
 // coefficients and every turn taking every kind of step; a 346x260 window 0.69 ms against 1.40.
 template <int kMaxG, bool kOne>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void cascade_walk_kernel(const CameraDev* cams, int n_cams, uint32_t n_total,
-                                                           const uint32_t* order, unsigned int* queue, WalkTuning tu,
-                                                           const CallDev* call) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void cascade_walk_kernel(
+    const CameraDev* cams, int n_cams, uint32_t n_total, const uint32_t* order, unsigned int* queue, const CallDev* call) {
   if (call_refused(cams, n_cams)) return;
   cascade_lanes<kMaxG, kOne>(cams, n_cams, n_total, order, queue, call->t_end);
 }
@@ -1587,6 +1586,11 @@ hipError_t launch_chain_walk(const ChainArgs& a, hipStream_t stream) {
     if (a.n_cams == 1) BSX_WALK(K, G, true);  \
     else BSX_WALK(K, G, false);               \
   } while (0)
+#define BSX_CASCADE(K, G)                                                                                          \
+  do {                                                                                                             \
+    if (a.n_cams == 1) K<G, true><<<grid, block, 0, stream>>>(a.cams, a.n_cams, a.n_total, a.perm, a.queue, a.call); \
+    else K<G, false><<<grid, block, 0, stream>>>(a.cams, a.n_cams, a.n_total, a.perm, a.queue, a.call);             \
+  } while (0)
 #define BSX_TIERS(LAUNCH, K)       \
   do {                             \
     if (tier == 0) LAUNCH(K, 1);   \
@@ -1596,8 +1600,9 @@ hipError_t launch_chain_walk(const ChainArgs& a, hipStream_t stream) {
   } while (0)
   if (a.instant) BSX_TIERS(BSX_LANES, instant_walk_kernel);
   else if (a.noise) BSX_TIERS(BSX_WALK, noise_walk_kernel);
-  else BSX_TIERS(BSX_LANES, cascade_walk_kernel);
+  else BSX_TIERS(BSX_CASCADE, cascade_walk_kernel);
 #undef BSX_TIERS
+#undef BSX_CASCADE
 #undef BSX_LANES
 #undef BSX_WALK
   return hipGetLastError();

@@ -5,6 +5,8 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
+#include <utility>
+#include <vector>
 
 namespace bsx {
 
@@ -159,28 +161,37 @@ std::vector<RigTrial> Rig::autotune(const bsx_device_runs* runs, int64_t t_end_n
     trials.push_back(RigTrial{tu, best});
     return best;
   };
-  // Coordinate descent: each axis in turn, every value, the best kept; two passes.
-  static const int kBlocks[] = {64, 128, 256};
-  static const int kBudgets[] = {4, 8, 16, 32, 64};
-  static const int kBatches[] = {1, 4, 8, 16, 32, 64};
-  static const int kChunks[] = {0, 1, 2, 4, 8, 16};
-  // The head (lanes, thousandths of the order): none, or the heaviest pixels in groups of 16 or 32.
-  static const int kHeads[][2] = {{64, 0}, {16, 8}, {32, 8}, {32, 32}};
+  // Coordinate descent: each axis in turn, every value, the best kept; two passes. The axes are those the walk
+  // reads (WalkTuning): of the cascade's without noise the block alone, of the instantaneous one the block, the
+  // budget, the batch and the lanes that refill together, of the one with in-path noise the block, the groups per grab
+  // and the head.
+  using Set = std::vector<std::pair<int32_t WalkTuning::*, int32_t>>;  // one value of an axis
+  const auto axis_of = [](int32_t WalkTuning::*field, std::initializer_list<int32_t> values) {
+    std::vector<Set> axis;
+    for (const int32_t v : values) axis.push_back(Set{{field, v}});
+    return axis;
+  };
+  std::vector<std::vector<Set>> axes{axis_of(&WalkTuning::block, {64, 128, 256})};
+  if (instant) {
+    axes.push_back(axis_of(&WalkTuning::walk_budget, {1, 2, 4, 8, 16}));
+    axes.push_back(axis_of(&WalkTuning::search_batch, {1, 2, 4, 8, 16, 64}));
+    axes.push_back(axis_of(&WalkTuning::chunk, {0, 8, 16, 32, 64}));
+  } else if (cds[0].kc.noise.tab != nullptr) {
+    axes.push_back(axis_of(&WalkTuning::chunk, {0, 1, 2, 4, 8, 16}));
+    // the head (lanes, thousandths of the order): none, or the heaviest pixels in groups of 16 or 32
+    std::vector<Set> head;
+    for (const auto& h : {std::pair{64, 0}, {16, 8}, {32, 8}, {32, 32}})
+      head.push_back(Set{{&WalkTuning::head_lanes, h.first}, {&WalkTuning::head_per_mille, h.second}});
+    axes.push_back(head);
+  }
   WalkTuning best = chain_.tuning();
   double best_ms = time_walk(best);
   for (int pass = 0; pass < 2; ++pass) {
-    for (int axis = 0; axis < 5; ++axis) {
-      const int* vals = axis == 0 ? kBlocks : axis == 1 ? kBudgets : axis == 2 ? kBatches : kChunks;
-      const int nv = axis == 0 ? 3 : axis == 1 ? 5 : axis == 4 ? 4 : 6;
+    for (const std::vector<Set>& axis : axes) {
       const WalkTuning base = best;
-      for (int k = 0; k < nv; ++k) {
+      for (const Set& values : axis) {
         WalkTuning t = base;
-        if (axis == 4) {
-          t.head_lanes = kHeads[k][0];
-          t.head_per_mille = kHeads[k][1];
-        } else {
-          (axis == 0 ? t.block : axis == 1 ? t.walk_budget : axis == 2 ? t.search_batch : t.chunk) = vals[k];
-        }
+        for (const auto& [field, v] : values) t.*field = v;
         const double ms = time_walk(t);
         if (ms < best_ms) {
           best_ms = ms;

@@ -35,9 +35,9 @@ class Rig {
   // uninitialized.
   void advance_device(const bsx_device_runs* runs, int64_t t_end_ns, hipStream_t stream, bsx_device_events* out);
 
-  // Times the walk of the given call under candidate tunings (coordinate descent over block size,
-  // walk budget, search batch and queue chunk from the current tuning, `reps` timed walks per
-  // candidate, minimum taken), keeps the fastest and returns the trials. No camera changes.
+  // Times the walk of the given call under candidate tunings (coordinate descent over the fields that the
+  // cameras' walk reads from the current tuning, `reps` timed walks per candidate, minimum taken), keeps the
+  // fastest and returns the trials. No camera changes.
   std::vector<RigTrial> autotune(const bsx_device_runs* runs, int64_t t_end_ns, hipStream_t stream, int reps);
 
   LaunchChain& chain() { return chain_; }

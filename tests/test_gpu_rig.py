@@ -21,6 +21,8 @@ def _params(kind, **over):
         p.noise = False
         p.leak_rate_hz = 0.5
         p.refractory_s = 5e-5
+    elif kind == "noise":
+        p = bsx.preset("prophesee_gen3")
     else:
         p = bsx.preset("samsung_gen3")
         p.noise = False
@@ -196,6 +198,32 @@ def test_rig_autotune_changes_no_camera():
         for k in want:
             assert np.array_equal(have[k], want[k]), (c, k)
         assert cams[c].save_state() == solo[c].save_state()
+
+
+# The fields each kind of walk reads, and values of them that must be among the candidates.
+@pytest.mark.parametrize("kind,live", [
+    ("instant", dict(block_size={64, 128, 256}, walk_budget={1, 2, 4, 8}, search_batch={1, 2, 4}, queue_chunk={0, 32, 64})),
+    ("cascade", dict(block_size={64, 128, 256})),
+    ("noise", dict(block_size={64, 128, 256}, queue_chunk={0, 1, 16}, head_lanes={64, 16, 32}, head_per_mille={0, 8, 32})),
+])
+def test_rig_autotune_tries_what_the_walk_reads(kind, live):
+    import torch
+
+    import ballasim_amd as bsx
+    rng = np.random.default_rng(7)
+    shapes = [(24, 16), (17, 9)]
+    cams = make_cameras(kind, shapes)
+    for c, (W, H) in enumerate(shapes):
+        cams[c].init(0, np.exp(rng.normal(3, 1, (W * H, 1))).astype(np.float32))
+    rig = bsx.Rig(cams)
+    runs = [to_device(*heavy_runs(rng, W * H, 0, 2 ** 21)) for (W, H) in shapes]
+    torch.cuda.synchronize()
+    base = rig.tuning()
+    trials = [t for t, _ in rig.autotune(runs, 2 ** 21, reps=1)]
+    assert len({tuple(sorted(t.items())) for t in trials}) == len(trials)  # no shape twice
+    for f in base:
+        seen = {t[f] for t in trials}
+        assert seen >= live[f] if f in live else seen == {base[f]}, (f, seen)
 
 
 def test_rig_refusals_change_no_camera():
