@@ -133,22 +133,39 @@ def test_rig_instant_without_graph_and_persistent_queue():
     assert rig.stats()["graph_launches"] == 0
 
 
+# Head groups and the queue of 64-pixel groups, which the walk with in-path noise takes: groups that divide the head,
+# leave a remainder, cover the whole order or more groups than a grab.
 @pytest.mark.parametrize("graph,tuning", [
     (True, dict(head_lanes=16, head_per_mille=250)),
     (False, dict(head_lanes=8, head_per_mille=500, queue_chunk=2, block_size=128)),
+    (True, dict(head_lanes=7, head_per_mille=333, queue_chunk=1)),
+    (True, dict(head_lanes=1, head_per_mille=1000, queue_chunk=64)),
+    (False, dict(queue_chunk=1, block_size=64)),
+    (True, dict(queue_chunk=3)),
 ])
-def test_rig_instant_head_groups(graph, tuning):
-    """The heaviest pixels of the order walked in groups of fewer than 64 (idle lanes in those waves)
-    give every camera the events, state and counters of advancing it alone in 64-pixel groups."""
-    rig, _ = run_pair("instant", SHAPES, graph=graph, tuning=tuning)
+def test_rig_noise_head_groups_and_queue(graph, tuning):
+    """The heaviest pixels of the order walked in groups of fewer than 64 (idle lanes in those waves), and groups taken
+    from the queue, give every camera the events, state and counters of advancing it alone in 64-pixel groups."""
+    rig, _ = run_pair("noise", [(24, 16), (17, 9)], calls=2, graph=graph, tuning=tuning)
     got = rig.tuning()
-    assert got["head_lanes"] == tuning["head_lanes"] and got["head_per_mille"] == tuning["head_per_mille"]
+    for f, v in tuning.items():
+        assert got[f] == v
     rig.set_tuning(head_per_mille=-1)
     assert rig.tuning()["head_per_mille"] == 0
 
 
-def test_rig_cascade_head_groups():
-    run_pair("cascade", [(24, 16), (17, 9)], calls=2, tuning=dict(head_lanes=32, head_per_mille=300))
+@pytest.mark.parametrize("kind,graph,tuning", [
+    ("instant", True, dict(head_lanes=16, head_per_mille=250)),
+    ("instant", False, dict(head_lanes=8, head_per_mille=500, queue_chunk=2, block_size=128)),
+    ("cascade", True, dict(head_lanes=32, head_per_mille=300)),
+])
+def test_rig_without_noise_takes_no_heads(kind, graph, tuning):
+    """The walks whose lanes take their pixels one by one accept the settings of the head, keep them, and read none."""
+    rig, _ = run_pair(kind, SHAPES if kind == "instant" else [(24, 16), (17, 9)], calls=2, graph=graph, tuning=tuning)
+    got = rig.tuning()
+    assert got["head_lanes"] == tuning["head_lanes"] and got["head_per_mille"] == tuning["head_per_mille"]
+    rig.set_tuning(head_per_mille=-1)
+    assert rig.tuning()["head_per_mille"] == 0
 
 
 def test_rig_cameras_at_different_times_and_overflow():
