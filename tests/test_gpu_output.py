@@ -3,6 +3,8 @@ reference's output_order / readout / label_s1): per window the released events, 
 every C4 column are identical, and the held count matches; with a crop and a readout with delay,
 quantum and clock offset and drift; then flush. Also the C4 file written from the released columns
 (t monotone, ms_to_idx)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -233,8 +235,6 @@ def test_columns_on_any_stream(kind):
 
 @pytest.mark.parametrize("missing", ["x", "t", "flags"])
 def test_fetch_refuses_a_null_column(missing):
-    import ctypes as C
-
     import torch
 
     import ballasim_amd as bsx
@@ -297,3 +297,54 @@ def test_bursts(burst, spread):
         for a, b in (("x", "x"), ("y", "y"), ("p", "p"), ("t_reported_ns", "t_reported"), ("t_cross_ns", "t_cross")):
             assert np.array_equal(got[a], want[b]), a
     assert stage.held == 0
+
+
+class OutputEvents(C.Structure):
+    """bsx_output_events: host columns owned by the stage."""
+    _fields_ = [("count", C.c_size_t), ("x", C.c_void_p), ("y", C.c_void_p), ("p", C.c_void_p), ("t", C.c_void_p),
+                ("t_ns_rem", C.c_void_p), ("t_reported_ns", C.c_void_p), ("t_cross_ns", C.c_void_p),
+                ("label", C.c_void_p), ("flags", C.c_void_p), ("held", C.c_size_t)]
+
+
+# bsx_output_window and bsx_output_flush, whose columns the stage itself holds, against the calls that fetch them: no
+# events, one staging chunk (of 1 MiB: 30,840 events), two, and several.
+@pytest.mark.parametrize("n", [0, 1, 30000, 50000, 150000])
+def test_columns_held_by_the_stage_equal_the_fetched(n):
+    import torch
+
+    import ballasim_amd as bsx
+    from ballasim_amd import _abi
+    from ballasim_amd.output import _COLUMNS, OutputStage
+    p = bsx.preset("prophesee_gen3")
+    p.photoreceptor = "instantaneous"
+    p.noise = False
+    p.readout_delay_s = 2e-3  # a quarter of the events is held for the flush
+    Wd, Hd = 640, 480
+    m = bsx.SensorModel(p, Wd, Hd, 3, ["constant"], 0, device="cuda")
+    rng = np.random.default_rng(n)
+    ev = np.zeros(n, RAW_EVENT)
+    ev["pixel"] = rng.integers(0, Wd * Hd, n)
+    ev["polarity"] = rng.integers(0, 2, n)
+    ev["label"] = rng.integers(0, 4, n)
+    ev["flags"] = rng.integers(0, 1 << 14, n)
+    ev["t_cross"] = 1 + rng.permutation(n) * (W // max(n, 1))
+    dev = torch.from_numpy(ev.view(np.uint8).reshape(n, 32)).cuda()
+    torch.cuda.synchronize()
+    fetched, own = OutputStage(m, t_offset_us=17), OutputStage(m, t_offset_us=17)
+    lib = _abi.load_library()
+    events = _abi.DeviceEvents(dev.data_ptr() if n else None, n)
+    for call in ("window", "flush"):
+        out = OutputEvents()
+        if call == "window":
+            want = fetched.window((dev.data_ptr() if n else 0, n), 0)
+            _abi.check(lib.bsx_output_window(own._h, C.byref(events), 0, None, C.byref(out)))
+        else:
+            want = fetched.flush()
+            _abi.check(lib.bsx_output_flush(own._h, None, C.byref(out)))
+        assert out.count == len(want["t"]) and out.held == fetched.held
+        assert n < 100 or out.count > n // 8  # both calls release events
+        for name, dt in _COLUMNS:
+            got = np.zeros(0, dt)
+            if out.count:
+                got = np.frombuffer(C.string_at(getattr(out, name), out.count * np.dtype(dt).itemsize), dt)
+            assert np.array_equal(got, want[name]), (call, name)
