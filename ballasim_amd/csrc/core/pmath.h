@@ -99,7 +99,8 @@ BSX_HD BSX_INLINE double frexp_exact(double x, int* e) {
 // reciprocal of b rounded to nearest and q0 near a / b, the remainder r = a - b q0 is exact in one fused
 // multiply-add and q0 + r y rounds to a / b (Markstein, IBM J. Res. Dev. 34 (1990) 111), away from
 // overflow and underflow. A function of one argument that uses these forms is compared with plain
-// divisions over every fp32 argument (bsx_math_hash). On the host they are plain divisions.
+// divisions over every fp32 argument its callers can reach, and div_with over 2^32 drawn pairs (bsx_math_hash).
+// On the host they are plain divisions.
 
 // a / kC for a small integer constant, whose reciprocal is a constant. The same bits as a / kC for |a| in
 // [2^-100, 2^100]; a smaller |a| may differ in its last bit, a zero in its sign, an infinity gives NaN.
