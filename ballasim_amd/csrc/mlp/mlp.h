@@ -49,8 +49,8 @@ hipError_t launch_gradients(const uint16_t* wb, const float* b_fp32, const float
 // fp32 masters w (moments m, v) and their bf16 copies wb.
 hipError_t launch_adam(const float* partial, int partials, float* grad, float* w, float* m, float* v, uint16_t* wb,
                        const Adam& a, hipStream_t stream);
-// MFMA check: C [32 x 32] fp32 = A [32 x 8] . B [8 x 32], A and B bf16 row-major, through the kernels'
-// tile routine (a self-check of the operand layouts).
+// MFMA check: C [32 x 32] fp32 = A [32 x 8] . B [8 x 32], A and B bf16 row-major, through each of
+// the kernels' matrix instructions (a self-check of the operand layouts).
 hipError_t launch_tile_check(const uint16_t* a, const uint16_t* b, float* c, hipStream_t stream);
 
 }  // namespace mlp

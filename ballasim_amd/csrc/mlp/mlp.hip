@@ -1,6 +1,6 @@
-// Kernels of the learned proposer: bf16 copies, batched forward, per-group gradients (forward and
-// backward on the MFMA units, four waves per group of 64 rows), and the reduction of the partial
-// gradients with an Adam step.
+// Kernels of the learned proposer: bf16 copies, batched forward, gradients (forward and backward on the
+// MFMA units, four waves of a block on 64 rows each at a time, one partial gradient per block), and the
+// reduction of the partial gradients with an Adam step.
 #include <hip/hip_runtime.h>
 
 #include "mlp_dev.h"
@@ -31,8 +31,17 @@ __device__ __forceinline__ f32x16 mma(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// The hidden unit of element i of k-chunk c for the lanes of half h.
-__device__ __forceinline__ int unit_of(int c, int h, int i) { return 16 * c + 8 * (i >> 2) + 4 * h + (i & 3); }
+// The hidden unit of element i of k-chunk c for the lanes of half h: the unit of accumulator element 8 (c % 2) + i of
+// tile c / 2.
+__host__ __device__ constexpr int unit_of(int c, int h, int i) { return 16 * c + 8 * (i >> 2) + 4 * h + (i & 3); }
+constexpr bool unit_of_matches_accumulators() {
+  for (int c = 0; c < 4; ++c)
+    for (int h = 0; h < 2; ++h)
+      for (int i = 0; i < 8; ++i)
+        if (unit_of(c, h, i) != 32 * (c >> 1) + acc_row_of(8 * (c & 1) + i, h)) return false;
+  return true;
+}
+static_assert(unit_of_matches_accumulators());
 
 __device__ __forceinline__ __bf16 bits_bf16(uint16_t u) { return __builtin_bit_cast(__bf16, u); }
 
@@ -429,16 +438,39 @@ __global__ __launch_bounds__(32 * kAdamSlices) void adam_kernel(const float* par
   wb[i] = to_bf16(wi);
 }
 
+// A . B (32x8 by 8x32) as the mean of the three matrix instructions that the kernels issue, each with all its k slots
+// filled (two and four copies of the eight products) and read back as the kernels read it: an operand or accumulator
+// taken from the wrong lane in any of them shows.
 __global__ __launch_bounds__(64) void tile_check_kernel(const uint16_t* a, const uint16_t* b, float* c) {
-  __shared__ uint16_t as[32 * 8], bs[8 * 32];
-  for (int i = threadIdx.x; i < 256; i += 64) {
-    as[i] = a[i];
-    bs[i] = b[i];
+  __shared__ float quarter[32 * 32];
+  const int l = threadIdx.x, r = l & 31, h = l >> 5;
+  bf16x4 a4, b4;  // the learned sampler's
+  bf16x8 a8, b8;  // forward and gradients, k in the order of unit_of
+  for (int i = 0; i < 4; ++i) {
+    a4[i] = static_cast<short>(a[r * 8 + 4 * h + i]);
+    b4[i] = static_cast<short>(b[(4 * h + i) * 32 + r]);
   }
+  for (int i = 0; i < 8; ++i) {
+    const int k = unit_of(0, h, i) & 7;
+    a8[i] = bits_bf16(a[r * 8 + k]);
+    b8[i] = bits_bf16(b[k * 32 + r]);
+  }
+  for (int m0 = 0; m0 < 32; m0 += 16)
+    for (int n0 = 0; n0 < 32; n0 += 16) {  // the bias sums'
+      bf16x8 at, bt;
+      for (int i = 0; i < 8; ++i) {
+        at[i] = bits_bf16(a[(m0 + (l & 15)) * 8 + i]);
+        bt[i] = bits_bf16(b[i * 32 + n0 + (l & 15)]);
+      }
+      const f32x4 q = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at, bt, f32x4{}, 0, 0, 0);
+      for (int j = 0; j < 4; ++j) quarter[(m0 + 4 * (l >> 4) + j) * 32 + n0 + (l & 15)] = 0.25f * q[j];
+    }
   __syncthreads();
-  f32x16 acc = {};
-  mma_tile(acc, as, 8, 1, bs, 32, 1, 8);
-  for (int j = 0; j < 16; ++j) c[acc_row(j) * 32 + acc_col()] = acc[j];
+  const f32x16 one = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a4, b4, f32x16{}, 0, 0, 0), two = mma(a8, b8, f32x16{});
+  for (int j = 0; j < 16; ++j) {
+    const int at = acc_row(j) * 32 + acc_col();
+    c[at] = (one[j] + 0.5f * two[j] + quarter[at]) / 3.0f;
+  }
 }
 
 }  // namespace

@@ -1,11 +1,11 @@
-// Device building blocks of the proposer's kernels: bf16 rounding, the 32x32 MFMA tile over operands
-// in LDS, and the forward pass of one wave's 64 rows (used by the training kernel and the learned
-// sampler).
+// Device building blocks of the proposer's kernels: bf16 rounding, the layout of the 32x32 MFMA accumulators, the
+// weights in LDS, and the learned sampler's forward pass of one wave's 64 rows (training and inference have their own
+// in mlp.hip).
 //
 // MFMA: v_mfma_f32_32x32x8bf16_1k multiplies a 32x8 bf16 tile A by an 8x32 bf16 tile B into a 32x32
 // fp32 accumulator. Lane l (of 64) supplies A[l % 32][4 (l / 32) + i] and B[4 (l / 32) + i][l % 32]
 // for i = 0..3, and holds accumulator element j (of 16) at row 8 (j / 4) + 4 (l / 32) + j % 4,
-// column l % 32. (launch_tile_check tests this layout against a host product.)
+// column l % 32. (launch_tile_check tests the kernels' matrix instructions against a host product.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -40,24 +40,9 @@ __device__ __forceinline__ void wave_sync() {
 
 __device__ __forceinline__ float silu(float z) { return z / (1.0f + __expf(-z)); }
 
-// acc += A . B over k = 0 .. K - 1 (K a multiple of 8) for the 32x32 tile whose A rows start at a and
-// B columns at b: A(m, k) = a[m * am + k * ak], B(k, n) = b[k * bk + n * bn] (bf16 in LDS). Called by
-// all 64 lanes of the wave.
-__device__ __forceinline__ void mma_tile(f32x16& acc, const uint16_t* a, int am, int ak, const uint16_t* b, int bk,
-                                         int bn, int K) {
-  const int l = threadIdx.x & 63, r = l & 31, kq = (l >> 5) * 4;
-  for (int k0 = 0; k0 < K; k0 += 8) {
-    bf16x4 av, bv;
-    for (int i = 0; i < 4; ++i) {
-      av[i] = static_cast<short>(a[r * am + (k0 + kq + i) * ak]);
-      bv[i] = static_cast<short>(b[(k0 + kq + i) * bk + r * bn]);
-    }
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(av, bv, acc, 0, 0, 0);
-  }
-}
-
-// Row and column of accumulator element j of this lane.
-__device__ __forceinline__ int acc_row(int j) { return 8 * (j >> 2) + 4 * ((threadIdx.x & 63) >> 5) + (j & 3); }
+// Row and column of accumulator element j of this lane (row: of the lanes of half h).
+__host__ __device__ constexpr int acc_row_of(int j, int h) { return 8 * (j >> 2) + 4 * h + (j & 3); }
+__device__ __forceinline__ int acc_row(int j) { return acc_row_of(j, (threadIdx.x & 63) >> 5); }
 __device__ __forceinline__ int acc_col() { return threadIdx.x & 31; }
 
 // The weights as the kernels hold them in LDS: bf16 matrices (W1 padded to 16 input rows) and fp32

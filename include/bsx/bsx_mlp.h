@@ -44,7 +44,7 @@ int bsx_mlp_train(bsx_mlp* m, const float* x, const float* target, int64_t n, in
 /* y [n] (device) = the network's output for the n device rows x [n x 12]. */
 int bsx_mlp_predict(bsx_mlp* m, const float* x, int64_t n, float* y, void* stream);
 /* Self-check of the MFMA operand layout: c [32 x 32] = a [32 x 8] . b [8 x 32] (host arrays, a and b
- * bf16 bit patterns, row-major) through the kernels' tile routine on the device. */
+ * bf16 bit patterns, row-major) through the matrix instructions that the kernels use, on the device. */
 int bsx_mlp_tile_check(const uint16_t* a, const uint16_t* b, float* c);
 
 /* ---- Training examples and the learned sampler -------------------------------------------------------
