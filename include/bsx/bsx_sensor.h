@@ -216,8 +216,8 @@ int bsx_device_count(int32_t* out);
 int bsx_math_selfcheck(uint64_t* log_violations, uint64_t* log_hash);
 /* Test aid: an order-independent hash of the device's results of one fp32 function (by number: log, exp,
  * erfcx, dawson, the residual exponentials of orders 1 to 4, 1/x, x/3, x/6, x/384, 1/x by recip, and div_with on a
- * pair drawn from the pattern) over the bit patterns
- * first, first + stride, ... <= last. No reference counterpart. */
+ * pair drawn from the pattern) over the bit patterns first, first + stride, ... <= last. No reference
+ * counterpart. */
 int bsx_math_hash(int32_t fn, uint32_t first, uint32_t last, uint32_t stride, uint64_t* hash);
 
 /* Reference: preset(name), src/sensor/params.h:176; preset_names(), :177 (names joined by ','). */
