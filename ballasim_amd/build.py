@@ -45,6 +45,9 @@ DEVICE = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-fhip-fp32-correctly-rounded-divide-sqrt",
 ]
+# Functions start at 64-byte lines: where they fell by the sizes of the code before them, the host's loops over a call's
+# samples and events took 2.8 or 3.4 ms of a 173x131 call by changes in other files alone.
+HOST = ["--offload-host-only", "-falign-functions=64"]
 
 
 def hipcc():
@@ -60,7 +63,7 @@ def _compile(src):
     if src.endswith(".hip"):
         cmd += DEVICE + ["-x", "hip"]
     else:
-        cmd += DEVICE + ["--offload-host-only"]  # host code only: the kernels live in the .hip files
+        cmd += DEVICE + HOST  # host code only: the kernels live in the .hip files
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")

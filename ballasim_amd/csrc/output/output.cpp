@@ -46,8 +46,6 @@ OutputStage::OutputStage(uint32_t width, uint32_t height, const Readout& readout
 OutputStage::~OutputStage() {
   if (h_scratch_ != nullptr) (void)hipHostFree(h_scratch_);
   if (staging_ != nullptr) (void)hipHostFree(staging_);
-  if (columns_ready_ != nullptr) (void)hipEventDestroy(columns_ready_);
-  if (copy_ != nullptr) (void)hipStreamDestroy(copy_);
 }
 
 void OutputStage::read_scratch(hipStream_t stream) {
@@ -187,12 +185,12 @@ constexpr int kCopySlots = 2 * kCopyThreads;
 // pages fault in as it writes (2.9 M events, 98 MB of columns: 13-17 ms with a second copy by the caller). Here
 // each of a few threads copies its chunks to pinned slots of its own and from there to their places, the next
 // chunk's transfer under way meanwhile, so that the transfers, the copies and the page faults overlap. Up to two
-// slots' bytes the calling thread does it alone. The threads' transfers go out on a stream of the stage's own, behind
-// an event the calling thread records on the caller's stream: a handle like hipStreamPerThread names another stream
-// in each thread, on which a transfer would not wait for the columns.
+// slots' bytes the calling thread does it alone, and so it does where the caller names its stream by
+// hipStreamPerThread: that handle is another stream in each thread, on which a transfer would not wait for the columns.
 void OutputStage::copy_out(const char* from, const std::vector<Piece>& dst, size_t bytes, hipStream_t stream) {
   const size_t chunks = (bytes + kCopyBytes - 1) / kCopyBytes;
-  const int slots = chunks <= 2 ? 2 : kCopySlots;
+  const bool alone = chunks <= 2 || stream == hipStreamPerThread;
+  const int slots = alone ? 2 : kCopySlots;
   if (slots > staging_slots_) {
     if (staging_ != nullptr) hip_check(hipHostFree(staging_), "staging");
     staging_ = nullptr;
@@ -214,16 +212,16 @@ void OutputStage::copy_out(const char* from, const std::vector<Piece>& dst, size
     place(0, staging_, bytes);
     return;
   }
-  const auto run = [&](size_t first, size_t step, char* slots, hipStream_t queue) {
+  const auto run = [&](size_t first, size_t step, char* slots) {
     hipEvent_t landed[2] = {nullptr, nullptr};
     hipError_t e = hipEventCreateWithFlags(&landed[0], hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&landed[1], hipEventDisableTiming);
     const auto size_of = [&](size_t c) { return std::min(kCopyBytes, bytes - c * kCopyBytes); };
     const auto start = [&](size_t c, int s) {
       if (e == hipSuccess) {
-        e = hipMemcpyAsync(slots + s * kCopyBytes, from + c * kCopyBytes, size_of(c), hipMemcpyDeviceToHost, queue);
+        e = hipMemcpyAsync(slots + s * kCopyBytes, from + c * kCopyBytes, size_of(c), hipMemcpyDeviceToHost, stream);
       }
-      if (e == hipSuccess) e = hipEventRecord(landed[s], queue);
+      if (e == hipSuccess) e = hipEventRecord(landed[s], stream);
     };
     int s = 0;
     if (first < chunks) start(first, s);
@@ -233,28 +231,22 @@ void OutputStage::copy_out(const char* from, const std::vector<Piece>& dst, size
       if (e == hipSuccess) place(c * kCopyBytes, slots + s * kCopyBytes, size_of(c));
     }
     // (after an error a transfer may still be writing the slots)
-    if (e != hipSuccess) (void)hipStreamSynchronize(queue);
+    if (e != hipSuccess) (void)hipStreamSynchronize(stream);
     for (hipEvent_t& ev : landed)
       if (ev != nullptr) (void)hipEventDestroy(ev);
     return e;
   };
-  if (chunks <= 2) {
-    hip_check(run(0, 1, staging_, stream), "download columns");
+  if (alone) {
+    hip_check(run(0, 1, staging_), "download columns");
     return;
   }
-  if (copy_ == nullptr) hip_check(hipStreamCreateWithFlags(&copy_, hipStreamNonBlocking), "copy stream");
-  if (columns_ready_ == nullptr) {
-    hip_check(hipEventCreateWithFlags(&columns_ready_, hipEventDisableTiming), "event create");
-  }
-  hip_check(hipEventRecord(columns_ready_, stream), "event record");
-  hip_check(hipStreamWaitEvent(copy_, columns_ready_, 0), "columns");
   int device = 0;
   hip_check(hipGetDevice(&device), "device");
   const size_t n_threads = std::min<size_t>(kCopyThreads, (chunks + 1) / 2);
   std::atomic<int> error{hipSuccess};
   run_workers(n_threads, [&](size_t k) noexcept {
     hipError_t e = hipSetDevice(device);
-    if (e == hipSuccess) e = run(k, n_threads, staging_ + 2 * k * kCopyBytes, copy_);
+    if (e == hipSuccess) e = run(k, n_threads, staging_ + 2 * k * kCopyBytes);
     if (e != hipSuccess) error.store(e);
   });
   hip_check(static_cast<hipError_t>(error.load()), "download columns");

@@ -118,8 +118,6 @@ class OutputStage {
   unsigned long long* h_scratch_ = nullptr;  // pinned
   char* staging_ = nullptr;             // pinned: staging_slots_ slots of kCopyBytes
   int staging_slots_ = 0;
-  hipStream_t copy_ = nullptr;            // of the copying threads' transfers
-  hipEvent_t columns_ready_ = nullptr;    // on the caller's stream, behind the columns
   OutputColumns out_;
 };
 
