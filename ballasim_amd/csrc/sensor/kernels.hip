@@ -641,6 +641,30 @@ __device__ __forceinline__ void camera_add(const CameraDev* cams, int cam_index,
   }
 }
 
+// The work counters of a walk whose lanes take pixels of several cameras in turn: summed per camera in the block's
+// LDS as the pixels finish (kN counters, words[k] of the camera's) and added to the cameras' at the walk's end. (One
+// wave reduction and global atomic per camera and counter at every refill took 0.09 of a four-camera rig's 0.95-ms
+// walk.) begin and end are called by every thread of the block, add by the finished lanes.
+constexpr int kMaxLaunchCameras = 64;
+template <int kN>
+struct RigTally {
+  unsigned long long* sums;  // LDS, [n_cams][kN]
+  int n_cams;
+
+  __device__ __forceinline__ void begin() const {
+    for (int i = threadIdx.x; i < n_cams * kN; i += blockDim.x) sums[i] = 0;
+    __syncthreads();
+  }
+  __device__ __forceinline__ void add(int ci, int k, uint32_t v) const {
+    if (v != 0) atomicAdd(sums + ci * kN + k, static_cast<unsigned long long>(v));
+  }
+  __device__ __forceinline__ void end(const CameraDev* cams, const int (&words)[kN]) const {
+    __syncthreads();
+    for (int i = threadIdx.x; i < n_cams * kN; i += blockDim.x)
+      if (sums[i] != 0) atomicAdd(cams[i / kN].counters + 1 + words[i % kN], sums[i]);
+  }
+};
+
 // The pixels a wave's lanes take in turn: positions of the launch's heavy-first order. With a queue the grid
 // is resident and persistent: the first pixels are dealt out one per wave, wave after wave, so that the
 // heaviest lie in different waves, and later ones are taken from the queue. Without one each lane takes the
@@ -771,11 +795,13 @@ __device__ __forceinline__ void instant_store(InstantLane<kMaxG>& L, const Camer
   out.shot_index[p] = L.shot_index;
 }
 
-template <int kMaxG>
-__device__ __forceinline__ void instant_count(const CameraDev* cams, int ci, InstantLane<kMaxG>& L) {
-  camera_add(cams, ci, 1 + kStSubsteps, L.n_substeps);
-  camera_add(cams, ci, 1 + kStPieces, L.n_pieces);
-  camera_add(cams, ci, 1 + kStLeaves, L.n_leaves);
+// add(k, v): the lane's count k, in the order of kInstantWords, is v.
+__device__ constexpr int kInstantWords[3] = {kStSubsteps, kStPieces, kStLeaves};
+template <int kMaxG, class Add>
+__device__ __forceinline__ void instant_counts(const InstantLane<kMaxG>& L, const Add& add) {
+  add(0, L.n_substeps);
+  add(1, L.n_pieces);
+  add(2, L.n_leaves);
 }
 
 // The instantaneous walk. The wave's lanes walk their pixels; a lane that reaches an exact search waits until
@@ -796,20 +822,24 @@ __device__ __forceinline__ void instant_lanes(const CameraDev* cams, int n_cams,
   Lane L;
   L.n_substeps = L.n_pieces = L.n_leaves = 0;
   int mode = kIdle, ci = -1, p = 0;
+  __shared__ unsigned long long sums[kOne ? 1 : kMaxLaunchCameras * 3];
+  const RigTally<3> tally{sums, n_cams};
   if constexpr (kOne) instant_constants(L, cams);
+  else tally.begin();
   while (true) {
     if (mode == Lane::kDone) mode = kIdle;
     const int idle = __popcll(__ballot(mode == kIdle)), searching = __popcll(__ballot(mode == Lane::kSearch)),
               walking = __popcll(__ballot(mode == Lane::kWalk));
     if (idle + searching + walking == 0) break;
     if (idle > 0 && (searching + walking == 0 || feed.exhausted || idle >= refill)) {
-      // save the finished pixels and take new ones (a rig's counters are kept per pixel, as the next one's
-      // camera may be another)
-      const bool done = mode == kIdle && ci >= 0;
-      if (done) instant_store(L, kOne ? cams : cams + ci, p);
-      if constexpr (!kOne) {
-        instant_count(cams, done ? ci : -1, L);
-        if (done) L.n_substeps = L.n_pieces = L.n_leaves = 0;
+      // save the finished pixels and take new ones (a rig's counts go to the pixel's camera, as the next one's may
+      // be another)
+      if (mode == kIdle && ci >= 0) {
+        instant_store(L, kOne ? cams : cams + ci, p);
+        if constexpr (!kOne) {
+          instant_counts(L, [&](int k, uint32_t v) { tally.add(ci, k, v); });
+          L.n_substeps = L.n_pieces = L.n_leaves = 0;
+        }
       }
       const uint32_t i = feed.take(mode == kIdle);
       if (mode == kIdle) {
@@ -837,7 +867,8 @@ __device__ __forceinline__ void instant_lanes(const CameraDev* cams, int n_cams,
       mode = L.walk(sink, tu.walk_budget);
     }
   }
-  if constexpr (kOne) instant_count(cams, 0, L);
+  if constexpr (kOne) instant_counts(L, [&](int k, uint32_t v) { camera_add(cams, 0, 1 + kInstantWords[k], v); });
+  else tally.end(cams, kInstantWords);
 }
 
 // The walk's groups over n pixels of the heavy-first order: tu.head_groups groups of tu.head_lanes
@@ -1037,15 +1068,18 @@ __device__ __forceinline__ void cascade_store(CascadeLane<kMaxG>& L, const Camer
 }
 
 // The lanes' work counters into their cameras' (every lane of the wave calls it; ci < 0: none).
-template <int kMaxG>
-__device__ __forceinline__ void cascade_count(const CameraDev* cams, int ci, CascadeLane<kMaxG>& L) {
-  camera_add(cams, ci, 1 + kStSubsteps, L.n_substeps);
-  camera_add(cams, ci, 1 + kStAttempts, L.n_attempts);
-  camera_add(cams, ci, 1 + kStSettled, L.n_settled);
-  camera_add(cams, ci, 1 + kStLeaves, L.n_leaves);
-  camera_add(cams, ci, 1 + kStFallbacks, L.n_fallbacks);
-  camera_add(cams, ci, 1 + kStQuarantines, L.n_quarantines);
-  camera_add(cams, ci, 1 + kStPieces, L.n_pieces);
+// add(k, v): the lane's count k, in the order of kCascadeWords, is v.
+__device__ constexpr int kCascadeWords[7] = {kStSubsteps, kStAttempts,    kStSettled, kStLeaves,
+                                             kStFallbacks, kStQuarantines, kStPieces};
+template <int kMaxG, class Add>
+__device__ __forceinline__ void cascade_counts(const CascadeLane<kMaxG>& L, const Add& add) {
+  add(0, L.n_substeps);
+  add(1, L.n_attempts);
+  add(2, L.n_settled);
+  add(3, L.n_leaves);
+  add(4, L.n_fallbacks);
+  add(5, L.n_quarantines);
+  add(6, L.n_pieces);
 }
 
 // The coefficients of the sub-step tries [0, h] with input Ia -> Ib that the lanes of `tries` are due
@@ -1155,7 +1189,10 @@ __device__ __forceinline__ void cascade_lanes(const CameraDev* cams, int n_cams,
   L.n_substeps = L.n_pieces = L.n_leaves = 0;
   L.n_attempts = L.n_settled = L.n_fallbacks = L.n_quarantines = 0;
   int state = kIdle, ci = -1, p = 0;
+  __shared__ unsigned long long sums[kOne ? 1 : kMaxLaunchCameras * 7];
+  const RigTally<7> tally{sums, n_cams};
   if constexpr (kOne) cascade_constants(L, cams);
+  else tally.begin();
   while (true) {
     if (state == Lane::kMove) {
       state = L.prepare();
@@ -1166,13 +1203,12 @@ __device__ __forceinline__ void cascade_lanes(const CameraDev* cams, int n_cams,
     const int busy = __popcll(__ballot(state > Lane::kFinished));
     if (idle + busy == 0) break;
     if (idle > 0 && (busy == 0 || feed.exhausted || idle >= kRefillLanes)) {
-      // save the finished pixels and take new ones (a rig's counters are kept per pixel, as the next one's
-      // camera may be another)
-      const bool done = state == kIdle && ci >= 0;
-      if (done) cascade_store(L, kOne ? cams : cams + ci, p);
-      if constexpr (!kOne) {
-        cascade_count(cams, done ? ci : -1, L);
-        if (done) {
+      // save the finished pixels and take new ones (a rig's counts go to the pixel's camera, as the next one's may
+      // be another)
+      if (state == kIdle && ci >= 0) {
+        cascade_store(L, kOne ? cams : cams + ci, p);
+        if constexpr (!kOne) {
+          cascade_counts(L, [&](int k, uint32_t v) { tally.add(ci, k, v); });
           L.n_substeps = L.n_pieces = L.n_leaves = 0;
           L.n_attempts = L.n_settled = L.n_fallbacks = L.n_quarantines = 0;
         }
@@ -1218,7 +1254,8 @@ __device__ __forceinline__ void cascade_lanes(const CameraDev* cams, int n_cams,
     }
     if (due) state = Lane::kMove;
   }
-  if constexpr (kOne) cascade_count(cams, 0, L);
+  if constexpr (kOne) cascade_counts(L, [&](int k, uint32_t v) { camera_add(cams, 0, 1 + kCascadeWords[k], v); });
+  else tally.end(cams, kCascadeWords);
 }
 
 // Bound by VALU issue and by the heaviest pixels' chains of steps. The helpers are inlined into the lane
@@ -1574,6 +1611,7 @@ int chain_walk_blocks(const ChainArgs& a) {
 }
 
 hipError_t launch_chain_walk(const ChainArgs& a, hipStream_t stream) {
+  if (a.n_cams > kMaxLaunchCameras) return hipErrorInvalidValue;
   const hipError_t e = chain_check(a);
   if (e != hipSuccess) return e;
   if (a.n_total == 0) return hipSuccess;
