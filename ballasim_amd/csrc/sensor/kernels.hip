@@ -666,25 +666,27 @@ struct RigTally {
 };
 
 // The pixels a wave's lanes take in turn: positions of the launch's heavy-first order. With a queue the grid
-// is resident and persistent: the first pixels are dealt out one per wave, wave after wave, so that the
-// heaviest lie in different waves, and later ones are taken from the queue. Without one each lane takes the
-// pixel of its place.
+// is resident and persistent: the first pixels are dealt out one per wave, wave after wave, to `deal` lanes of
+// each, so that the heaviest lie in different waves, and later ones are taken from the queue. Without one each lane
+// takes the pixel of its place.
 struct LaneFeed {
+  static constexpr uint32_t kNone = 0xffffffffu, kLater = 0xfffffffeu;
   uint32_t n_total, wave, n_waves, dealt;
   unsigned int* queue;
   bool begun = false, exhausted = false;  // (uniform over the wave)
 
-  __device__ __forceinline__ LaneFeed(uint32_t n, unsigned int* q) : n_total(n), queue(q) {
+  __device__ __forceinline__ LaneFeed(uint32_t n, unsigned int* q, uint32_t deal) : n_total(n), queue(q) {
     n_waves = gridDim.x * (blockDim.x / 64);
     wave = (blockIdx.x * blockDim.x + threadIdx.x) / 64;
     const uint32_t each = (n + n_waves - 1) / n_waves;
-    dealt = (each < 64 ? each : 64) * n_waves;
+    dealt = (each < deal ? each : deal) * n_waves;
   }
 
-  // Positions for the `wants` lanes (past n_total: none). Called by every lane of the wave.
+  // Positions for the `wants` lanes (kLater: none yet, ask again; past n_total otherwise: none). Called by every
+  // lane of the wave.
   __device__ __forceinline__ uint32_t take(bool wants) {
     const uint32_t lane = __lane_id();
-    if (exhausted) return 0xffffffffu;
+    if (exhausted) return kNone;
     if (queue == nullptr) {
       exhausted = true;
       return wave * 64 + lane;
@@ -692,7 +694,7 @@ struct LaneFeed {
     if (!begun) {
       begun = true;
       exhausted = dealt >= n_total;
-      return lane * n_waves < dealt ? lane * n_waves + wave : 0xffffffffu;
+      return lane * n_waves < dealt ? lane * n_waves + wave : exhausted ? kNone : kLater;
     }
     const unsigned long long waiting = __ballot(wants);
     uint32_t first = 0;
@@ -810,7 +812,10 @@ __device__ __forceinline__ void instant_counts(const InstantLane<kMaxG>& L, cons
 // Bound by the latency of the lanes' dependent steps: dealing the heaviest pixels one to a wave, where a wave of 64
 // of them set the walk's length, took a 1280x720 window's chain from 2.46 to 2.19 ms, a 2048x1536 window's from
 // 16.6 to 13.5 and a 64x48 call's from 0.36 to 0.23 (refill 8: 14.1 ms of 2048x1536, 16: 13.8, 48: 13.5, 64:
-// 14.2; walk_budget 1, 2, 4, 8: 14.8, 14.4, 13.5, 14.5; search_batch 2, 4, 16: 13.6, 13.5, 13.9).
+// 14.2; walk_budget 1, 2, 4, 8: 14.8, 14.4, 13.5, 14.5; search_batch 2, 4, 16: 13.6, 13.5, 13.9). Where most pixels
+// have little to do a whole wave of them is taken at once and few lanes are dealt the heavy ones (a four-camera rig
+// of 3.4 M pixels, launches with phase A's 1.92 ms: refill 48: 3.26 ms, 64: 2.95, deal 16, 8, 4, 2, 1 lanes: 2.93,
+// 2.92, 2.90, 2.88, 2.89).
 template <int kMaxG, bool kOne>
 __device__ __forceinline__ void instant_lanes(const CameraDev* cams, int n_cams, uint32_t n_total, const uint32_t* order,
                                               unsigned int* queue, const WalkTuning& tu, int64_t t_end,
@@ -818,7 +823,7 @@ __device__ __forceinline__ void instant_lanes(const CameraDev* cams, int n_cams,
   using Lane = InstantLane<kMaxG>;
   constexpr int kIdle = -1, kOut = -2;  // waiting for a pixel (the last one not saved yet); none left
   const int refill = tu.chunk > 0 ? tu.chunk : 48;  // idle lanes that take pixels together
-  LaneFeed feed(n_total, queue);
+  LaneFeed feed(n_total, queue, static_cast<uint32_t>(tu.head_per_mille > 0 ? tu.head_lanes : 64));
   Lane L;
   L.n_substeps = L.n_pieces = L.n_leaves = 0;
   int mode = kIdle, ci = -1, p = 0;
@@ -844,8 +849,8 @@ __device__ __forceinline__ void instant_lanes(const CameraDev* cams, int n_cams,
       const uint32_t i = feed.take(mode == kIdle);
       if (mode == kIdle) {
         ci = -1;
-        mode = kOut;
-        if (i < n_total) {
+        if (i != LaneFeed::kLater) mode = kOut;
+        if (i < n_total && i != LaneFeed::kLater) {
           const uint32_t g = order != nullptr ? order[i] : i;
           ci = kOne ? 0 : camera_of(cams, n_cams, g);
           const CameraDev* cam = kOne ? cams : cams + ci;
@@ -1184,7 +1189,7 @@ __device__ __forceinline__ void cascade_lanes(const CameraDev* cams, int n_cams,
                                               unsigned int* queue, int64_t t_end) {
   using Lane = CascadeLane<kMaxG>;
   constexpr int kIdle = -1, kOut = -2;  // waiting for a pixel (the last one not saved yet); none left
-  LaneFeed feed(n_total, queue);
+  LaneFeed feed(n_total, queue, 64);
   Lane L;
   L.n_substeps = L.n_pieces = L.n_leaves = 0;
   L.n_attempts = L.n_settled = L.n_fallbacks = L.n_quarantines = 0;

@@ -154,18 +154,50 @@ def test_rig_noise_head_groups_and_queue(graph, tuning):
     assert rig.tuning()["head_per_mille"] == 0
 
 
+# The heads of the other walks: lanes of a wave dealt pixels before the queue (instantaneous: one, a few, with refills
+# that come at once, when a whole wave is idle, or never, as no pixels are left), and none (cascade).
 @pytest.mark.parametrize("kind,graph,tuning", [
     ("instant", True, dict(head_lanes=16, head_per_mille=250)),
     ("instant", False, dict(head_lanes=8, head_per_mille=500, queue_chunk=2, block_size=128)),
+    ("instant", True, dict(head_lanes=1, head_per_mille=8, queue_chunk=64)),
+    ("instant", True, dict(head_lanes=2, head_per_mille=8, queue_chunk=64, block_size=64)),
     ("cascade", True, dict(head_lanes=32, head_per_mille=300)),
 ])
-def test_rig_without_noise_takes_no_heads(kind, graph, tuning):
-    """The walks whose lanes take their pixels one by one accept the settings of the head, keep them, and read none."""
+def test_rig_heads_without_noise(kind, graph, tuning):
     rig, _ = run_pair(kind, SHAPES if kind == "instant" else [(24, 16), (17, 9)], calls=2, graph=graph, tuning=tuning)
     got = rig.tuning()
     assert got["head_lanes"] == tuning["head_lanes"] and got["head_per_mille"] == tuning["head_per_mille"]
     rig.set_tuning(head_per_mille=-1)
     assert rig.tuning()["head_per_mille"] == 0
+
+
+@pytest.mark.parametrize("head", [1, 2, 63])
+def test_lanes_dealt_and_from_the_queue(head):
+    """More pixels than the walk's resident waves, so that lanes that are dealt none take theirs from the queue."""
+    import torch
+
+    import ballasim_amd as bsx
+    rng = np.random.default_rng(head)
+    shapes = [(331, 97), (64, 9)]
+    cams, solo = make_cameras("instant", shapes), make_cameras("instant", shapes)
+    for c, (W, H) in enumerate(shapes):
+        irr0 = np.exp(rng.normal(3, 1, (W * H, 1))).astype(np.float32)
+        cams[c].init(0, irr0)
+        solo[c].init(0, irr0)
+    rig = bsx.Rig(cams)
+    rig.set_tuning(head_lanes=head, head_per_mille=8, queue_chunk=64)
+    t_end = 2 ** 21
+    runs = [to_device(*heavy_runs(rng, W * H, 0, t_end, mu=np.log(2.0), cap=40)) for (W, H) in shapes]
+    torch.cuda.synchronize()
+    got = rig.advance_device(runs, t_end)
+    for c in range(len(shapes)):
+        ptr, count = solo[c].advance_device(*runs[c], t_end)
+        want, have = solo[c].download_events(ptr, count), cams[c].download_events(*got[c])
+        for k in want:
+            assert np.array_equal(have[k], want[k]), (c, k)
+        assert cams[c].save_state() == solo[c].save_state()
+        for k in WORK:
+            assert cams[c].stats()[k] == solo[c].stats()[k], (c, k)
 
 
 def test_rig_cameras_at_different_times_and_overflow():
@@ -219,7 +251,8 @@ def test_rig_autotune_changes_no_camera():
 
 # The fields each kind of walk reads, and values of them that must be among the candidates.
 @pytest.mark.parametrize("kind,live", [
-    ("instant", dict(block_size={64, 128, 256}, walk_budget={1, 2, 4, 8}, search_batch={1, 2, 4}, queue_chunk={0, 32, 64})),
+    ("instant", dict(block_size={64, 128, 256}, walk_budget={4, 8}, search_batch={1, 2, 4}, queue_chunk={0, 32, 64},
+                     head_lanes={64, 8, 2}, head_per_mille={0, 8})),
     ("cascade", dict(block_size={64, 128, 256})),
     ("noise", dict(block_size={64, 128, 256}, queue_chunk={0, 1, 16}, head_lanes={64, 16, 32}, head_per_mille={0, 8, 32})),
 ])
