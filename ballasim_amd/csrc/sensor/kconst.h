@@ -164,11 +164,11 @@ struct CallDev {
 };
 
 // The walk's launch shape, chosen by the autotuner: threads per block and, for the instantaneous walk,
-// segments a walking lane does before the wave looks again, waiting lanes that start a joint search, idle lanes
-// that take pixels from the queue together (chunk; 0: 48) and, if head_per_mille is set, the lanes of a wave that
-// are dealt the heaviest pixels (head_lanes; else all). The walk with in-path noise takes its pixels 64 at a time:
-// chunk is the groups a wave takes per grab of the queue (0: one group per wave, no queue), and the head of
-// the heavy-first order may be walked in groups of fewer than 64 pixels.
+// segments a walking lane does before the wave looks again, waiting lanes that start a joint search, whether a
+// wave takes pixels from the queue 64 at a time (chunk > 0) or as 48 of its lanes are idle and, if head_per_mille is
+// set, the lanes of a wave that are dealt the heaviest pixels (head_lanes; else all). The walk with in-path noise
+// takes its pixels 64 at a time: chunk is the groups a wave takes per grab of the queue (0: one group per wave, no
+// queue), and the head of the heavy-first order may be walked in groups of fewer than 64 pixels.
 struct WalkTuning {
   int32_t block;
   int32_t walk_budget;

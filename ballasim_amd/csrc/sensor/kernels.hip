@@ -822,7 +822,7 @@ __device__ __forceinline__ void instant_lanes(const CameraDev* cams, int n_cams,
                                               uint32_t* stacks) {
   using Lane = InstantLane<kMaxG>;
   constexpr int kIdle = -1, kOut = -2;  // waiting for a pixel (the last one not saved yet); none left
-  const int refill = tu.chunk > 0 ? tu.chunk : 48;  // idle lanes that take pixels together
+  const int refill = tu.chunk > 0 ? 64 : 48;  // idle lanes that take pixels together
   LaneFeed feed(n_total, queue, static_cast<uint32_t>(tu.head_per_mille > 0 ? tu.head_lanes : 64));
   Lane L;
   L.n_substeps = L.n_pieces = L.n_leaves = 0;

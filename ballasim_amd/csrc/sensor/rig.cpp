@@ -163,8 +163,8 @@ std::vector<RigTrial> Rig::autotune(const bsx_device_runs* runs, int64_t t_end_n
   };
   // Coordinate descent: each axis in turn, every value, the best kept; two passes. The axes are those the walk
   // reads (WalkTuning): of the cascade's without noise the block alone, of the instantaneous one the block, the
-  // budget, the batch, the lanes that refill together and those that are dealt to, of the one with in-path noise the
-  // block, the groups per grab and the head. (Budgets below 4: as the lanes dealt to below, by 3 %.)
+  // budget, the batch, how pixels are taken from the queue and the lanes that are dealt to, of the one with in-path
+  // noise the block, the groups per grab and the head. (Budgets below 4: as the lanes dealt to below, by 3 %.)
   using Set = std::vector<std::pair<int32_t WalkTuning::*, int32_t>>;  // one value of an axis
   const auto axis_of = [](int32_t WalkTuning::*field, std::initializer_list<int32_t> values) {
     std::vector<Set> axis;
@@ -181,12 +181,12 @@ std::vector<RigTrial> Rig::autotune(const bsx_device_runs* runs, int64_t t_end_n
   if (instant) {
     axes.push_back(axis_of(&WalkTuning::walk_budget, {4, 8, 16}));
     axes.push_back(axis_of(&WalkTuning::search_batch, {1, 2, 4, 8, 16, 64}));
-    // the lanes that refill together and, where a whole wave does, those that are dealt to (with earlier refills a
-    // few lanes dealt to won on a first, heavy window and lost 2 % over the run)
-    std::vector<Set> refill = heads({{64, 0}, {64, 0}, {64, 0}, {64, 0}, {64, 0}, {8, 8}, {2, 8}});
-    const int32_t lanes[] = {0, 8, 16, 32, 64, 64, 64};
-    for (size_t k = 0; k < refill.size(); ++k) refill[k].push_back({&WalkTuning::chunk, lanes[k]});
-    axes.push_back(refill);
+    // single pixels or whole waves from the queue and, with whole waves, the lanes that are dealt to (with single
+    // pixels a few lanes dealt to won on a first, heavy window and lost 2 % over the run)
+    std::vector<Set> take = heads({{64, 0}, {64, 0}, {8, 8}, {2, 8}});
+    const int32_t chunks[] = {0, 1, 1, 1};
+    for (size_t k = 0; k < take.size(); ++k) take[k].push_back({&WalkTuning::chunk, chunks[k]});
+    axes.push_back(take);
   } else if (cds[0].kc.noise.tab != nullptr) {
     axes.push_back(axis_of(&WalkTuning::chunk, {0, 1, 2, 4, 8, 16}));
     axes.push_back(heads({{64, 0}, {16, 8}, {32, 8}, {32, 32}}));  // none, or the heaviest pixels in groups of 16 or 32

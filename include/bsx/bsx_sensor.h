@@ -179,12 +179,13 @@ typedef struct bsx_launch_policy {
   int32_t block_size;   /* threads per workgroup, a multiple of 64 in [64, 256] (default 256) */
   int32_t walk_budget;  /* segments a walking lane does before its wave re-plans, [1, 1024] (default 4) */
   int32_t search_batch; /* waiting lanes that start a joint exact-search pass, [1, 64] (default 4) */
-  int32_t queue_chunk;  /* [0, 64], -1 sets 0 (default 0). Instantaneous response: idle lanes of a wave that
-                           take pixels from the work queue together, 0 = 48. In-path noise: 64-pixel groups
-                           per grab of the queue, 0 = no queue. The cascade's lanes take theirs by a rule of
-                           its own. */
+  int32_t queue_chunk;  /* 64-pixel groups per grab of the work queue, [0, 64]; -1 sets 0 (default 0). Instantaneous
+                           response: from 1 on a wave takes 64 pixels at a time, with 0 its lanes take single
+                           ones, 48 together. In-path noise: 0 = no queue. The cascade's lanes take theirs by a
+                           rule of its own. */
   int32_t head_lanes;     /* in-path noise: pixels a walk group takes at the head of the heavy-first pixel
-                             order, [1, 64] (default 64) */
+                             order, [1, 64] (default 64). Instantaneous response, if head_per_mille > 0: lanes of
+                             a wave that are dealt the heaviest pixels */
   int32_t head_per_mille; /* the head's share of the order, in thousandths of the pixels, [0, 1000]; -1 sets
                              0 (default 0: every group takes 64 pixels) */
 } bsx_launch_policy;

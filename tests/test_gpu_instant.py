@@ -82,16 +82,16 @@ def test_instant_matches_oracle(case):
 
 # One pixel, one fewer and one more than a wave (and than the lanes that refill together), and more pixels than
 # the walk's resident lanes (256 CUs x 12 waves x 64), so that lanes take theirs from the queue; the launch
-# shapes that refill at every idle lane and at a whole wave of them.
+# shapes that refill at 48 idle lanes and at a whole wave of them.
 @pytest.mark.parametrize("W,H,frac", [(1, 1, 1.0), (47, 1, 1.0), (63, 1, 1.0), (65, 1, 0.9), (641, 331, 0.1)])
-@pytest.mark.parametrize("refill", [0, 1, 64])
-def test_lanes_take_pixels(W, H, frac, refill):
+@pytest.mark.parametrize("chunk", [0, 1, 64])
+def test_lanes_take_pixels(W, H, frac, chunk):
     import ballasim_amd as bsx
     rng = np.random.default_rng(W)
     p = _params("physical_leak")
     gpu = bsx.SensorModel(p, W, H, 5, ["constant"], 0, device="cuda")
-    if refill:
-        gpu.set_launch_policy(queue_chunk=refill)
+    if chunk:
+        gpu.set_launch_policy(queue_chunk=chunk)
     ref = O.OracleModel(p.c, W, H, 5, 1, 0)
     irr0 = np.exp(rng.normal(3, 1, size=(W * H, 1))).astype(np.float32)
     gpu.init(0, irr0)

@@ -155,7 +155,7 @@ def test_rig_noise_head_groups_and_queue(graph, tuning):
 
 
 # The heads of the other walks: lanes of a wave dealt pixels before the queue (instantaneous: one, a few, with refills
-# that come at once, when a whole wave is idle, or never, as no pixels are left), and none (cascade).
+# at 48 idle lanes or a whole wave), and none (cascade).
 @pytest.mark.parametrize("kind,graph,tuning", [
     ("instant", True, dict(head_lanes=16, head_per_mille=250)),
     ("instant", False, dict(head_lanes=8, head_per_mille=500, queue_chunk=2, block_size=128)),
@@ -251,7 +251,7 @@ def test_rig_autotune_changes_no_camera():
 
 # The fields each kind of walk reads, and values of them that must be among the candidates.
 @pytest.mark.parametrize("kind,live", [
-    ("instant", dict(block_size={64, 128, 256}, walk_budget={4, 8}, search_batch={1, 2, 4}, queue_chunk={0, 32, 64},
+    ("instant", dict(block_size={64, 128, 256}, walk_budget={4, 8}, search_batch={1, 2, 4}, queue_chunk={0, 1},
                      head_lanes={64, 8, 2}, head_per_mille={0, 8})),
     ("cascade", dict(block_size={64, 128, 256})),
     ("noise", dict(block_size={64, 128, 256}, queue_chunk={0, 1, 16}, head_lanes={64, 16, 32}, head_per_mille={0, 8, 32})),
