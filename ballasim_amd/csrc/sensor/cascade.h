@@ -768,8 +768,8 @@ struct CascadeLane : InstantLane<kMaxG, 2> {
   }
 
   // The sub-steps of one linear piece in nested loops, each followed by the comparator (cmp(sub): the
-  // noise lane's tree comparator). The same steps in the same order as piece_begin, piece_prepare and
-  // piece_attempt; the noise lane keeps its loops, which hold its state in fewer registers.
+  // noise lane's tree comparator). The same steps in the same order as prepare and attempt; the noise lane
+  // keeps its loops, which hold its state in fewer registers.
   template <class Cmp>
   BSX_HD BSX_INLINE void run_piece(const cascade::Piece& pc, Cmp&& cmp) {
     int64_t t_a = pc.t_a, h_hint = 0;

@@ -1,6 +1,7 @@
-// gfx950 kernels of the sensor path: init, the instantaneous-response advance, the input checks and
-// the run scatter. One lane per pixel; a 64-lane wave covers 64 consecutive pixels, so every state,
-// map and row-index access is one coalesced vector access; events leave through a wave-aggregated
+// gfx950 kernels of the sensor path: init, the advance's phase A, pixel order and walks (instantaneous,
+// cascade, cascade with in-path noise), the input checks and the run scatter. A lane walks a pixel; the
+// pixels come in heavy-first order, so a wave's lanes hold pixels from anywhere in the frame and their state,
+// map and run accesses are gathers (init's and the checks' are coalesced). Events leave through a wave-aggregated
 // sink (one atomic per wave and push site, consecutive slots for the active lanes).
 #include <hip/hip_runtime.h>
 
@@ -1277,8 +1278,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 
 // The cascade with its in-path noise: lane i of the launch's pixel order takes pixel order[i] of its
 // camera and advances it to t_end; mid is the lane's column of the tree walk's path memory (LDS). (Run
-// as machines in one loop, as cascade_lane runs its lanes, the noise walk measured no faster: 103 ms
-// against 100 ms on the first 1280x720 windows, with 576 bytes of scratch a lane against 432.)
+// as machines in one loop, a try per lane and turn, the noise walk measured no faster: 103 ms against 100 ms on
+// the first 1280x720 windows, with 576 bytes of scratch a lane against 432. Turns by kind of step, as cascade_lanes
+// takes them, have not been tried here.)
 template <int kMaxG>
 __device__ __forceinline__ void noise_lane(const CameraDev* cams, int n_cams, uint32_t n_total, const uint32_t* order,
                                            uint32_t i, int64_t t_end, float* mid, int mid_stride) {
