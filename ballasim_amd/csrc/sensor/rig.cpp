@@ -200,7 +200,7 @@ std::vector<RigTrial> Rig::autotune(const bsx_device_runs* runs, int64_t t_end_n
         WalkTuning t = base;
         for (const auto& [field, v] : values) t.*field = v;
         const double ms = time_walk(t);
-        if (ms < 0.995 * best_ms) {  // (a difference the timing shows again)
+        if (ms < best_ms) {
           best_ms = ms;
           best = t;
         }

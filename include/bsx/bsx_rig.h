@@ -59,9 +59,8 @@ int bsx_rig_stats(bsx_rig* rig, bsx_rig_stats_t* out);
  * reads are tried: block size {64, 128, 256}; for the instantaneous response also walk budget {4 .. 16},
  * search batch {1 .. 64}, queue chunk {0, 1} and, with 1, the head (64, 8 or 2 lanes); with in-path noise
  * also queue chunk {0 .. 16} and the head (64 lanes, or the heaviest 0.8 % or 3.2 % of the pixels by 16 or
- * 32). A shape is changed for one that is at least half a percent faster. No camera's state or
- * time changes (the cameras' event buffers are overwritten). Up to max_trials trials are returned
- * (tunings[i], walk_ms[i]; either pointer may be null), their count in *n_trials. */
+ * 32). No camera's state or time changes (the cameras' event buffers are overwritten). Up to max_trials
+ * trials are returned (tunings[i], walk_ms[i]; either pointer may be null), their count in *n_trials. */
 int bsx_rig_autotune(bsx_rig* rig, const bsx_device_runs* runs, int64_t t_end_ns, void* stream, int32_t reps,
                      bsx_launch_policy* tunings, double* walk_ms, int32_t max_trials, int32_t* n_trials);
 
